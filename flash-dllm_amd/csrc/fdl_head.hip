@@ -1,5 +1,5 @@
 // Confidence of the LM-head rows (gfx950): the float64 softmax maximum and its token, or
-// the float64 softmax probability of a given token, one pass of reads per row.
+// the float64 softmax probability of a given token, one workgroup per row.
 //
 // Replaces, for bf16 logits,
 //   p = softmax(logits.to(float64), -1); x0_p, x0 = max(p, -1)        (generate.py:218, :320)
@@ -19,7 +19,9 @@
 namespace fdl {
 namespace {
 
-constexpr int kConfThreads = 256;  // one workgroup per row
+constexpr int kConfThreads = 1024;  // one workgroup per row
+constexpr int kConfWaves = kConfThreads / kWave;
+constexpr int kDirectThreads = 256;
 
 __device__ __forceinline__ float bf16_lo(uint32_t w) { return __builtin_bit_cast(float, w << 16); }
 __device__ __forceinline__ float bf16_hi(uint32_t w) {
@@ -34,13 +36,14 @@ __device__ __forceinline__ void arg_max_merge(float& m, int64_t& i, float m2, in
   }
 }
 
-// vocab % 8 == 0 and 16-byte aligned rows (checked on the host).
-__global__ __launch_bounds__(kConfThreads) void softmax_conf_kernel(
+// vocab below kTableVocab: every exponential computed. vocab % 8 == 0 and 16-byte aligned rows
+// (checked on the host).
+__global__ __launch_bounds__(kDirectThreads) void softmax_conf_direct_kernel(
     const uint16_t* __restrict__ logits, int64_t vocab, const int64_t* __restrict__ token,
     double* __restrict__ prob, int64_t* __restrict__ arg) {
-  __shared__ float s_m[kConfThreads / kWave];
-  __shared__ int64_t s_i[kConfThreads / kWave];
-  __shared__ double s_sum[kConfThreads / kWave];
+  __shared__ float s_m[kDirectThreads / kWave];
+  __shared__ int64_t s_i[kDirectThreads / kWave];
+  __shared__ double s_sum[kDirectThreads / kWave];
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const uint16_t* x = logits + int64_t(blockIdx.x) * vocab;
   const int64_t n8 = vocab / 8;
@@ -49,7 +52,7 @@ __global__ __launch_bounds__(kConfThreads) void softmax_conf_kernel(
   // that visits none keeps the index past every real one)
   float m = -INFINITY;
   int64_t im = INT64_MAX;
-  for (int64_t c = tid; c < n8; c += kConfThreads) {
+  for (int64_t c = tid; c < n8; c += kDirectThreads) {
     const u32x4 v = ld16(x + 8 * c);
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
@@ -78,12 +81,12 @@ __global__ __launch_bounds__(kConfThreads) void softmax_conf_kernel(
   m = s_m[0];
   im = s_i[0];
 #pragma unroll
-  for (int w = 1; w < kConfThreads / kWave; ++w) arg_max_merge(m, im, s_m[w], s_i[w]);
+  for (int w = 1; w < kDirectThreads / kWave; ++w) arg_max_merge(m, im, s_m[w], s_i[w]);
 
   // pass 2: float64 sum of exp(x - m); per-thread partials, then a fixed reduction tree
   const double md = static_cast<double>(m);
   double s = 0.0;
-  for (int64_t c = tid; c < n8; c += kConfThreads) {
+  for (int64_t c = tid; c < n8; c += kDirectThreads) {
     const u32x4 v = ld16(x + 8 * c);
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
@@ -98,7 +101,203 @@ __global__ __launch_bounds__(kConfThreads) void softmax_conf_kernel(
   if (tid == 0) {
     double sum = s_sum[0];
 #pragma unroll
-    for (int w = 1; w < kConfThreads / kWave; ++w) sum += s_sum[w];
+    for (int w = 1; w < kDirectThreads / kWave; ++w) sum += s_sum[w];
+    double p;
+    if (token) {
+      const int64_t t = token[blockIdx.x];
+      p = t >= 0 && t < vocab ? exp(static_cast<double>(bf2f(x[t])) - md) / sum : 0.0;
+    } else {
+      p = 1.0 / sum;
+    }
+    prob[blockIdx.x] = p;
+    // A row with a NaN (no comparison above selects it, but it makes the sum NaN), a +inf or
+    // only -inf logits has a softmax of NaNs; torch.max of it returns index 0.
+    if (arg) arg[blockIdx.x] = __builtin_isfinite(m) && sum == sum ? im : 0;
+  }
+}
+
+// ---- vocab from kTableVocab on
+//
+// What bounds the row: 126464 float64 exponentials by one workgroup are far more work than its
+// 253 KB of reads (64 us of the 70 us at 256 rows when each is computed), and a second read of
+// the row comes from the Infinity Cache. bf16 logits have few distinct values, so the
+// exponentials of the common ones are tabulated once per row in LDS (4096 per row instead of
+// 126464) and summed by look-up, and the row stays in registers between the passes: 256 rows
+// of 126464 70 -> 24 us, 32 rows 58 -> 20 us, 512 rows of 32000 31 -> 20 us. What is left is
+// mostly the look-ups (bank conflicts of random 8-byte reads). Below 16384 values the table
+// costs more than it saves (512 rows of 8192: 10 us computed, 14 us tabulated; of 16384: 17
+// and 17 us; one row of 16384: 10 and 8 us), so shorter rows keep the direct kernel.
+constexpr int64_t kTableVocab = 16384;
+
+// exp(x - m) of the bf16 values with |x| in [2^-10, 2^6) (16 exponents, both signs) from a
+// table of float64 values made once per row: a bf16 of those exponents is its sign, the low
+// 4 bits of its exponent and its 7 fraction bits. Values outside (also 0, NaN, infinities)
+// take exp() itself.
+constexpr uint32_t kTabMagLo = 117u << 7;  // bits of 2^-10
+constexpr uint32_t kTabMags = 16u << 7;
+constexpr int kTabSize = 2 * kTabMags;  // 4096 values, 32 KB
+
+// whether all 8 values of v are in the table (the smallest and the largest magnitude bits, two
+// 16-bit halves at a time)
+__device__ __forceinline__ bool in_table(u32x4 v) {
+  typedef uint16_t u16x2 __attribute__((ext_vector_type(2)));
+  u16x2 lo, hi;
+#pragma unroll
+  for (int j = 0; j < 4; ++j) {
+    const u16x2 mag = __builtin_bit_cast(u16x2, v[j] & 0x7fff7fffu);
+    lo = j ? __builtin_elementwise_min(lo, mag) : mag;
+    hi = j ? __builtin_elementwise_max(hi, mag) : mag;
+  }
+  return min(lo[0], lo[1]) >= kTabMagLo && max(hi[0], hi[1]) < kTabMagLo + kTabMags;
+}
+
+// sum of the table's exp(x_j - m) over the 8 values of v (any bits read inside the table)
+__device__ __forceinline__ double table_sum8(u32x4 v, const double* tab) {
+  double s0 = 0.0, s1 = 0.0;
+#pragma unroll
+  for (int j = 0; j < 4; ++j) {
+    const uint32_t w = v[j];
+    s0 += tab[(w & (kTabMags - 1)) | ((w >> 15) & 1u) * kTabMags];
+    s1 += tab[((w >> 16) & (kTabMags - 1)) | (w >> 31) * kTabMags];
+  }
+  return s0 + s1;
+}
+
+__device__ __forceinline__ double exp_sum8(u32x4 v, double md) {
+  double s = 0.0;
+#pragma unroll 1
+  for (int j = 0; j < 4; ++j) {
+    s += exp(static_cast<double>(bf16_lo(v[j])) - md);
+    s += exp(static_cast<double>(bf16_hi(v[j])) - md);
+  }
+  return s;
+}
+
+// vocab % 8 == 0 and 16-byte aligned rows (checked on the host). Thread t takes the 16-byte
+// chunks t, t + 1024, ..; with kChunks > 0 (vocab <= 8192 kChunks) they stay in registers, so
+// the row is read from memory once; with kChunks == 0 the second pass reads it again.
+template <int kChunks>
+__global__ __launch_bounds__(kConfThreads) void softmax_conf_kernel(
+    const uint16_t* __restrict__ logits, int64_t vocab, const int64_t* __restrict__ token,
+    double* __restrict__ prob, int64_t* __restrict__ arg) {
+  __shared__ double tab[kTabSize];
+  __shared__ float s_m[kConfWaves];
+  __shared__ int64_t s_i[kConfWaves];
+  __shared__ double s_sum[kConfWaves];
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const uint16_t* x = logits + int64_t(blockIdx.x) * vocab;
+  const int64_t n8 = vocab / 8;
+
+  // the maximum (a NaN is never it; it makes the sum NaN)
+  u32x4 reg[kChunks > 0 ? kChunks : 1];
+  float m = -INFINITY;
+  auto max8 = [&](u32x4 v) {
+#pragma unroll
+    for (int j = 0; j < 4; ++j) m = fmaxf(m, fmaxf(bf16_lo(v[j]), bf16_hi(v[j])));
+  };
+  if constexpr (kChunks > 0) {
+#pragma unroll
+    for (int i = 0; i < kChunks; ++i) {
+      const int64_t c = tid + int64_t(kConfThreads) * i;
+      reg[i] = ld16(x + 8 * min(c, n8 - 1));  // past the end: the last chunk, not summed
+    }
+#pragma unroll
+    for (int i = 0; i < kChunks; ++i) max8(reg[i]);
+  } else {
+#pragma unroll 4
+    for (int64_t c = tid; c < n8; c += kConfThreads) max8(ld16(x + 8 * c));
+  }
+  // the chunks stay packed between the passes (no widened copies are carried over)
+  auto repack = [&]() {
+#pragma unroll
+    for (int i = 0; i < (kChunks > 0 ? kChunks : 0); ++i) asm volatile("" : "+v"(reg[i]));
+  };
+  repack();
+  const float m_own = m;
+#pragma unroll
+  for (int off = 32; off >= 1; off >>= 1) m = fmaxf(m, __shfl_xor(m, off));
+  if (lane == 0) s_m[wave] = m;
+  __syncthreads();
+  m = s_m[0];
+#pragma unroll
+  for (int w = 1; w < kConfWaves; ++w) m = fmaxf(m, s_m[w]);
+  const double md = static_cast<double>(m);
+
+  // the table, and the first index of the maximum (only threads that hold it look)
+#pragma unroll 1
+  for (int i = 0; i < kTabSize / kConfThreads; ++i) {
+    const uint32_t t = tid + kConfThreads * i;
+    const uint32_t low = t & (kTabMags - 1);
+    // the magnitude of the range whose low 11 bits these are
+    const uint32_t mag = kTabMagLo + ((low - kTabMagLo) & (kTabMags - 1));
+    tab[t] = exp(static_cast<double>(bf2f(static_cast<uint16_t>(mag | (t / kTabMags) << 15))) - md);
+  }
+  int64_t im = INT64_MAX;
+  if (m_own == m) {
+    auto first8 = [&](u32x4 v, int64_t c) {
+#pragma unroll
+      for (int j = 3; j >= 0; --j) {
+        if (bf16_hi(v[j]) == m) im = min(im, 8 * c + 2 * j + 1);
+        if (bf16_lo(v[j]) == m) im = min(im, 8 * c + 2 * j);
+      }
+    };
+    if constexpr (kChunks > 0) {
+      int hit = 0;  // the first chunk with the maximum
+#pragma unroll
+      for (int i = kChunks - 1; i >= 0; --i) {
+        float top = -INFINITY;
+#pragma unroll
+        for (int j = 0; j < 4; ++j) top = fmaxf(top, fmaxf(bf16_lo(reg[i][j]), bf16_hi(reg[i][j])));
+        hit = top == m ? i : hit;
+      }
+      const int64_t c = min(tid + int64_t(kConfThreads) * hit, n8 - 1);
+      first8(ld16(x + 8 * c), c);
+    } else {
+      for (int64_t c = tid; c < n8; c += kConfThreads) first8(ld16(x + 8 * c), c);
+    }
+  }
+#pragma unroll
+  for (int off = 32; off >= 1; off >>= 1) im = min(im, __shfl_xor(im, off));
+  if (lane == 0) s_i[wave] = im;
+  __syncthreads();
+
+  // float64 sum of exp(x - m): per-thread partials, then a fixed reduction tree
+  repack();
+  double s = 0.0;
+  if constexpr (kChunks > 0) {
+    uint32_t rest = 0;  // this thread's chunks that are not all in the table
+#pragma unroll
+    for (int i = 0; i < kChunks; ++i) {
+      if (tid + int64_t(kConfThreads) * i < n8) {
+        if (in_table(reg[i]))
+          s += table_sum8(reg[i], tab);
+        else
+          rest |= 1u << i;
+      }
+      if (i % 2) __builtin_amdgcn_sched_barrier(0);  // 16 look-ups in flight
+    }
+    for (; rest; rest &= rest - 1) {
+      const int64_t c = tid + int64_t(kConfThreads) * __builtin_ctz(rest);
+      s += exp_sum8(ld16(x + 8 * c), md);
+    }
+  } else {
+    for (int64_t c = tid; c < n8; c += kConfThreads) {
+      const u32x4 v = ld16(x + 8 * c);
+      s += in_table(v) ? table_sum8(v, tab) : exp_sum8(v, md);
+    }
+  }
+#pragma unroll
+  for (int off = 32; off >= 1; off >>= 1) s += __shfl_xor(s, off);
+  if (lane == 0) s_sum[wave] = s;
+  __syncthreads();
+  if (tid == 0) {
+    double sum = s_sum[0];
+    im = s_i[0];
+#pragma unroll
+    for (int w = 1; w < kConfWaves; ++w) {
+      sum += s_sum[w];
+      im = min(im, s_i[w]);
+    }
     double p;
     if (token) {
       const int64_t t = token[blockIdx.x];
@@ -129,9 +328,16 @@ extern "C" int fdl_softmax_confidence(const void* logits, int64_t n_rows, int64_
   FDL_REQUIRE_PTR(logits);
   FDL_REQUIRE_PTR(prob);
   FDL_REQUIRE_ALIGNED(logits, 16);
-  hipLaunchKernelGGL(softmax_conf_kernel, dim3(static_cast<unsigned>(n_rows)),
-                     dim3(kConfThreads), 0, static_cast<hipStream_t>(stream),
-                     static_cast<const uint16_t*>(logits), vocab, token, prob, arg);
+  constexpr int64_t per_chunk = int64_t(8) * kConfThreads;  // values per chunk of a workgroup
+  const bool direct = vocab < kTableVocab;
+  auto* kernel = direct                    ? softmax_conf_direct_kernel
+                 : vocab <= 4 * per_chunk  ? softmax_conf_kernel<4>
+                 : vocab <= 16 * per_chunk ? softmax_conf_kernel<16>
+                                           : softmax_conf_kernel<0>;
+  hipLaunchKernelGGL(kernel, dim3(static_cast<unsigned>(n_rows)),
+                     dim3(direct ? kDirectThreads : kConfThreads), 0,
+                     static_cast<hipStream_t>(stream), static_cast<const uint16_t*>(logits), vocab,
+                     token, prob, arg);
   FDL_HIP_CHECK(hipGetLastError());
   return ok();
 }

@@ -61,3 +61,30 @@ def test_softmax_confidence_non_finite_rows_match_torch():
     assert torch.equal(got_i, ref_i), (got_i, ref_i)
     assert torch.isnan(got_p[:3]).all() and torch.isnan(ref_p[:3]).all()
     np.testing.assert_allclose(got_p[3:].numpy(), ref_p[3:].numpy(), rtol=1e-12)
+
+
+@pytest.mark.parametrize("vocab", [16376, 16384, 32768, 32776, 131072, 131080])
+@pytest.mark.parametrize("token", [False, True])
+def test_softmax_confidence_kernel_edges(vocab, token):
+    """The vocabulary sizes at which another kernel takes over (direct, tabulated with the row
+    in registers, tabulated with the row read twice), on rows that hold the edges of the
+    tabulated range of magnitudes ([2^-10, 2^6)) and values outside it: zeros, denormals,
+    -inf, large ones. The terms are the reference's to an ulp or two of float64 and only the
+    order of up to 131080 positive terms differs: 1e-12 relative."""
+    gen = torch.Generator().manual_seed(vocab)
+    x = (torch.randn(4, vocab, generator=gen) * 3.0).to(torch.bfloat16)
+    edge = torch.tensor([0.0, -0.0, 2.0**-10, -2.0**-10, 2.0**-10 * (1 - 2.0**-8), 1e-40, -1e-40,
+                         63.75, -63.75, -64.0, -700.0, -3e38, float("-inf")]).to(torch.bfloat16)
+    x[1, 40:40 + len(edge)] = edge
+    x[1, vocab - len(edge):] = edge
+    x[2] = (x[2].float() * 40.0).to(torch.bfloat16)  # most values past the table
+    x[3] = 0.0                                         # nothing in the table, all tied
+    tok = torch.tensor([vocab - 1, 41, int(x[2].argmax()), vocab])
+    p = F.softmax(x.double(), dim=-1)
+    ref_p, ref_i = torch.max(p, dim=-1)
+    if token:
+        ref_p = p.gather(1, tok.clamp(max=vocab - 1)[:, None]).view(-1)
+        ref_p[3] = 0.0
+    prob, arg = ops.softmax_confidence(x.to(DEV), tok.to(DEV) if token else None)
+    torch.testing.assert_close(prob.cpu(), ref_p, rtol=1e-12, atol=0)
+    assert torch.equal(arg.cpu(), ref_i)
