@@ -21,17 +21,20 @@
 // from LDS. A consumer never issues a global memory instruction, so its MFMA stream is
 // never held behind the texture-address queue. After the reduction the consumers stage the
 // fp32 sums in the (then free) stage memory and every wavefront rotates and writes 8-pair
-// groups with 16-byte stores. Two shapes, chosen by the number of rows:
+// groups with 16-byte stores. Two shapes, chosen by the number of rows (many rows run 256-row
+// tiles of another kernel, fdl_pair_gemm.h; see qkv_split):
 //  * more than 128 rows: 128 rows x 96 pairs, 4 stages of 40 KB (all of LDS). 512 rows give
 //    one tile per CU.
 //  * up to 128 rows (weight streaming, HBM-bound): 64 or 128 rows x 32 pairs (192 tiles at
 //    d_model 4096), 8 stages of 16 KB or 6 of 24 KB, so each workgroup keeps 5-7 weight
 //    steps in flight.
+#include <algorithm>
 #include <atomic>
 #include <type_traits>
 
 #include "fdl_device.h"
 #include "fdl_host.h"
+#include "fdl_pair_gemm.h"
 
 namespace fdl {
 namespace {
@@ -429,16 +432,40 @@ __global__ __launch_bounds__((4 + NPROD) * 64, 1) void qkv_pc_kernel(QkvArgs a) 
   for (int j = 0; j < kPer; ++j) grp[j].store(a);
 }
 
+// Epilogue of the 256-row tiles (fdl_pair_gemm.h).
+struct RopeEp {
+  QkvArgs a;
+  struct Row {
+    int dkv, rope;  // K/V row, sin/cos row (both below 2^31: the host checks); -1: not stored
+  };
+  __device__ __forceinline__ const uint16_t* wrow(int p, int hi) const {
+    const int pairs_per_mat = a.n_heads * kHalf;
+    const int mat = p / pairs_per_mat, rem = p - mat * pairs_per_mat;
+    return a.w[mat] + int64_t((rem >> 6) * kHeadDim + (rem & 63) + kHalf * hi) * a.d_model;
+  }
+  __device__ __forceinline__ Row row(int64_t r) const {
+    int64_t dq, dkv, rope;
+    row_dest(a, r, dq, dkv, rope);
+    return {static_cast<int>(dkv), static_cast<int>(rope)};
+  }
+  __device__ __forceinline__ void store(const Row& d, int64_t r, int p, const float* lo,
+                                        const float* hi) const {
+    const int pairs_per_mat = a.n_heads * kHalf;
+    const int mat = p / pairs_per_mat, rem = p - mat * pairs_per_mat;
+    EpGroup g;
+    g.load(a, lo, static_cast<int>(hi - lo), mat, rem,
+           d.rope < 0 ? -1 : (mat == 0 ? r : int64_t(d.dkv)), d.rope);
+    g.store(a);
+  }
+};
+
 }  // namespace
 }  // namespace fdl
 
 namespace fdl {
 namespace {
 
-// Launch plan by row count (measured on MI355X at d_model 4096): up to 128 rows the
-// projection streams the weights (32-pair tiles, 192 workgroups, 6-8 stages: 18.6 us at
-// 40 rows, 23 us at 128); above that the wide tiles keep the MFMAs fed (128 x 32-pair
-// tiles take 45 us at 192 rows against 36 us for the wide tiles).
+// A producer / consumer tile shape.
 struct QkvPlan {
   void (*kernel)(QkvArgs);
   int bm;       // rows per tile
@@ -451,12 +478,6 @@ constexpr int kPcBM = 128, kPcBP = 96;
 template <int BM, int BP, int NPROD, int STAGES>
 constexpr QkvPlan pc_plan() {
   return {qkv_pc_kernel<BM, BP, NPROD, STAGES>, BM, BP, PcShape<BM, BP, NPROD, STAGES>::kThreads};
-}
-
-QkvPlan qkv_plan(int64_t n_rows) {
-  if (n_rows <= 64) return pc_plan<64, 32, 4, 8>();
-  if (n_rows <= 128) return pc_plan<128, 32, 4, 6>();
-  return pc_plan<kPcBM, kPcBP, 4, 4>();
 }
 
 // Compute units of the current device (cached per device).
@@ -474,26 +495,58 @@ int device_cus() {
   return n;
 }
 
-// Rows handed to the weight-streaming kernel at the end of a producer/consumer launch: a
-// remainder of at most 64 rows that would otherwise open one more round of workgroups on
-// the device (one workgroup per CU). At 576 rows: 4 full tiles (one round, 54 us) plus a
-// 64-row stream (19 us) instead of 5 tiles in two rounds (~100 us).
-int64_t qkv_tail_rows(int64_t n_rows, int64_t n_pairs) {
-  if (n_rows <= kPcBM) return 0;
-  const int64_t tail = n_rows % kPcBM;
-  if (tail == 0 || tail > 64) return 0;
-  const int64_t per_mtile = n_pairs / kPcBP;
+// Rows of a call and the shapes that run them: the first `wide` on 256-row tiles, the next
+// `mid` on 128-row tiles, the rest (at most 128) streaming the weights.
+struct QkvSplit {
+  int64_t wide, mid;
+};
+
+// Up to 128 rows the projection streams the weights (32-pair tiles, 192 workgroups, 6-8 stages:
+// 18.6 us at 40 rows, 23 us at 128; 128 x 32-pair tiles take 45 us at 192 rows against 36 us
+// for the 128 x 96-pair ones). Beyond, two shapes feed the MFMAs: a round of 256-row tiles (80
+// us at d_model 4096, one workgroup per CU) covers as much as two rounds of 128-row tiles (47
+// us each), so whole rounds go to the 256-row tiles and a part of a round to what covers it
+// soonest: 512 rows to 128-row tiles (54 us; 256-row tiles fill half of the device and take
+// 75), 1024 rows to 256-row tiles (100 -> 86 us), 1536 rows a round of each (140 -> 130 us), 576
+// rows a round of 128-row tiles and a 64-row stream (69 us; 256-row tiles 76), 640 rows to
+// 256-row tiles (95 -> 76 us). The split with the smallest sum is taken; a launch counts as
+// kLaunchUs.
+constexpr int kWideRoundUs = 80, kMidRoundUs = 47, kLaunchUs = 4;
+constexpr int kStreamUs[2] = {17, 21};  // up to 64 rows, up to 128
+constexpr int kStreamRows = 128;
+
+QkvSplit qkv_split(int64_t n_rows, int64_t n_pairs) {
   const int64_t cus = device_cus();
-  const int64_t full = (n_rows / kPcBM) * per_mtile;
-  const bool new_round = (full + per_mtile + cus - 1) / cus > (full + cus - 1) / cus;
-  return new_round ? tail : 0;
+  auto rounds = [&](int64_t rows, int bm, int bp) {
+    return ((rows + bm - 1) / bm * (n_pairs / bp) + cus - 1) / cus;
+  };
+  auto cost = [&](const QkvSplit& s) {
+    const int64_t rest = n_rows - s.wide - s.mid;
+    int64_t c = 0;
+    if (s.wide) c += rounds(s.wide, kPgBM, kPgBP) * kWideRoundUs + kLaunchUs;
+    if (s.mid) c += rounds(s.mid, kPcBM, kPcBP) * kMidRoundUs + kLaunchUs;
+    if (rest) c += rounds(rest, kStreamRows, 32) * kStreamUs[rest > 64] + kLaunchUs;
+    return c;
+  };
+  if (n_rows <= kStreamRows) return {0, 0};
+  QkvSplit best = {n_rows, 0};
+  // wide tiles in whole, the rest on 128-row tiles with or without its last, partial tile (a
+  // rest of more than two rounds of 256-row tiles is never the better choice)
+  const int64_t whole = n_rows / kPgBM, two_rounds = 2 * (cus / (n_pairs / kPgBP) + 1);
+  for (int64_t q = std::max<int64_t>(0, whole - two_rounds); q <= whole; ++q) {
+    const int64_t wide = q * kPgBM, rest = n_rows - wide;
+    const int64_t full = rest / kPcBM * kPcBM;
+    for (const int64_t mid : {rest, full, rest <= kStreamRows ? 0 : rest}) {
+      const QkvSplit s = {wide, mid};
+      if (cost(s) < cost(best)) best = s;
+    }
+  }
+  return best;
 }
 
-// Launches `plan` over rows [r0, r0 + n) of the call described by `args`.
-hipError_t qkv_launch(const QkvPlan& plan, QkvArgs args, int64_t r0, int64_t n,
-                      hipStream_t stream) {
+// Rows [r0, r0 + n) of the call described by `args`.
+QkvArgs qkv_rows(QkvArgs args, int64_t r0, int64_t n) {
   const int64_t D = args.d_model;
-  const int64_t n_pairs = 3 * int64_t(args.n_heads) * kHalf;  // a multiple of every plan's bp
   args.x += r0 * D;
   args.slot += r0;
   if (args.rope_row) args.rope_row += r0;
@@ -504,13 +557,30 @@ hipError_t qkv_launch(const QkvPlan& plan, QkvArgs args, int64_t r0, int64_t n,
     args.n_kv_rows = n;
   }
   args.n_rows = n;
-  const int64_t n_mtiles = (n + plan.bm - 1) / plan.bm;
+  return args;
+}
+
+hipError_t qkv_launch(const QkvPlan& plan, QkvArgs args, hipStream_t stream) {
+  const int64_t n_pairs = 3 * int64_t(args.n_heads) * kHalf;  // a multiple of every plan's bp
+  const int64_t n_mtiles = (args.n_rows + plan.bm - 1) / plan.bm;
   const int64_t n_tiles = n_mtiles * (n_pairs / plan.bp);
   if (n_tiles >= (int64_t(1) << 31)) return hipErrorInvalidValue;
   args.n_mtiles = static_cast<int>(n_mtiles);
   args.n_tiles = static_cast<int>(n_tiles);
   hipLaunchKernelGGL(plan.kernel, dim3(static_cast<unsigned>(n_tiles)), dim3(plan.threads), 0,
                      stream, args);
+  return hipGetLastError();
+}
+
+hipError_t qkv_launch_wide(const QkvArgs& args, hipStream_t stream) {
+  const int64_t n_pairs = 3 * int64_t(args.n_heads) * kHalf;
+  const int64_t n_mtiles = (args.n_rows + kPgBM - 1) / kPgBM;
+  const int64_t n_tiles = n_mtiles * (n_pairs / kPgBP);
+  if (n_tiles >= (int64_t(1) << 31)) return hipErrorInvalidValue;
+  const PairGemmTiles t = {args.x, args.n_rows, args.d_model, static_cast<int>(n_mtiles),
+                           static_cast<int>(n_pairs / kPgBP)};
+  hipLaunchKernelGGL(pair_gemm_kernel<RopeEp>, dim3(static_cast<unsigned>(n_tiles)),
+                     dim3(kPgThreads), 0, stream, t, RopeEp{args});
   return hipGetLastError();
 }
 
@@ -590,9 +660,14 @@ extern "C" int fdl_qkv_rope_cache(const void* x, const void* wq, const void* wk,
   args.kv_packed = kv_packed;
   args.rope_half = (flags & FDL_QKV_ROPE_HALVES_EQUAL) ? 1 : 0;
   const hipStream_t st = static_cast<hipStream_t>(stream);
-  const int64_t tail = qkv_tail_rows(n_rows, 3 * n_heads * kHalf);
-  const int64_t head = n_rows - tail;
-  FDL_HIP_CHECK(qkv_launch(qkv_plan(head), args, 0, head, st));
-  if (tail > 0) FDL_HIP_CHECK(qkv_launch(qkv_plan(tail), args, head, tail, st));
+  const QkvSplit split = qkv_split(n_rows, 3 * n_heads * kHalf);
+  const int64_t rest = n_rows - split.wide - split.mid;
+  if (split.wide > 0) FDL_HIP_CHECK(qkv_launch_wide(qkv_rows(args, 0, split.wide), st));
+  if (split.mid > 0)
+    FDL_HIP_CHECK(qkv_launch(pc_plan<kPcBM, kPcBP, 4, 4>(),
+                             qkv_rows(args, split.wide, split.mid), st));
+  if (rest > 0)
+    FDL_HIP_CHECK(qkv_launch(rest <= 64 ? pc_plan<64, 32, 4, 8>() : pc_plan<128, 32, 4, 6>(),
+                             qkv_rows(args, split.wide + split.mid, rest), st));
   return ok();
 }

@@ -143,6 +143,48 @@ def test_qkv_packed_verify_mode(Q):
     _close(_np(v), v_ref, what="V packed")
 
 
+@pytest.mark.parametrize("kv_packed,halves", [(False, True), (True, False)])
+@pytest.mark.parametrize("heads,rows", [
+    (2, 8193),   # 4 reduction steps (the fewest), a last tile of one row
+    (4, 8192),   # one full round of 256-row tiles, tiles that straddle two matrices
+    (4, 8491),   # a round of 256-row tiles, the rest on 128-row tiles
+    (4, 8232),   # a round of 256-row tiles, the rest streamed
+    (4, 12304),  # a round of 256-row tiles, one of 128-row tiles, the rest streamed
+    (6, 2801),   # a tile count that is no multiple of 8
+])
+def test_qkv_rope_cache_many_rows(heads, rows, kv_packed, halves):
+    """Row counts that run 256-row tiles, alone and with a rest on another shape, equal bit for
+    bit to the same rows in calls of at most 500 (128-row tiles: the same products summed in
+    the same order); rows whose slot is out of range stay out of all three outputs."""
+    D = 128 * heads
+    gen = torch.Generator().manual_seed(rows)
+    n_slots = rows + 99
+    x = torch.randn(rows, D, generator=gen).to(torch.bfloat16).to(DEV)
+    w = [(torch.randn(D, D, generator=gen) * 0.05).to(torch.bfloat16).to(DEV) for _ in range(3)]
+    sin, cos = (torch.randn(n_slots, 128, generator=gen) for _ in range(2))
+    if halves:
+        sin[:, 64:], cos[:, 64:] = sin[:, :64], cos[:, :64]
+    sin, cos = sin.to(DEV), cos.to(DEV)
+    slot = torch.randperm(n_slots, generator=gen)[:rows]
+    slot[7], slot[rows - 1 if rows > 8300 else 300] = -1, n_slots
+    slot = slot.to(DEV)
+    n_kv = rows if kv_packed else n_slots
+
+    def outputs():
+        return [torch.full((n, D), POISON, dtype=torch.bfloat16, device=DEV)
+                for n in (rows, n_kv, n_kv)]
+
+    whole, parts = outputs(), outputs()
+    ops.qkv_rope_cache(x, *w, sin, cos, slot, *whole, heads, kv_packed=kv_packed)
+    for r in range(0, rows, 500):
+        kv = [t[r:r + 500] for t in parts[1:]] if kv_packed else parts[1:]
+        ops.qkv_rope_cache(x[r:r + 500], *w, sin, cos, slot[r:r + 500], parts[0][r:r + 500], *kv,
+                           heads, kv_packed=kv_packed)
+    for name, a, b in zip("QKV", whole, parts):
+        assert torch.equal(a, b), f"{name} differs"
+    assert bool((whole[0][7] == POISON).all()) and bool((whole[0][6] != POISON).any())
+
+
 # ------------------------------------------------------------------ block attention
 
 def _ref_tables(B, L, k_ends, masked_n, tracked):
