@@ -22,6 +22,7 @@
 // half-filled device gained, 76 -> 68 us at 512 rows).
 #pragma once
 
+#include <atomic>
 #include <type_traits>
 
 #include "fdl_device.h"
@@ -41,6 +42,9 @@ constexpr int kPgEpRows = 128;              // rows staged at a time
 static_assert(kPgEpRows * kPgEpStride * 4 <= kPgMetaOff, "epilogue staging");
 constexpr int kPgALoads = kPgABytes / 1024 / 8;  // 1 KB loads per wavefront and step
 constexpr int kPgBLoads = kPgBBytes / 1024 / 8;
+
+typedef __attribute__((address_space(3))) void* PgLds;
+typedef __attribute__((address_space(1))) void* PgGlb;
 
 struct PairGemmTiles {
   const uint16_t* x;  // [n_rows][k]
@@ -81,6 +85,284 @@ __device__ __forceinline__ void pg_wait() {
   asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory");
 }
 
+// Epilogue `Ep`: wrow(p, hi) is the first element of pair p's low or high weight row; row(r) ->
+// Ep::Row (8 bytes) says where output row r goes (also for r past n_rows: nowhere); Ep::Group
+// takes 8 consecutive pairs of one row: load(ep, row, r, p, lo, hi_off, mine) reads the low sums
+// at lo and the high sums at lo + hi_off (p a multiple of 8; nothing is stored unless mine),
+// store(ep) writes them.
+
+// ---------------------------------------------------------------------------------------
+// Producer / consumer tiles
+
+// LDS tile layout: chunk c (16 B) of tile row r is stored at chunk c ^ ((r >> 1) & 7) of
+// that row: two 128-byte rows share one 256-byte bank line, so 16 consecutive rows read at
+// the same logical chunk land on 16 distinct 4-bank groups.
+
+// Workgroup i runs on XCD i % 8. Renumber so that each XCD gets a contiguous run of tiles
+// (tiles are numbered n-block-major): the m-tiles that share one weight slice then run on
+// one XCD and share its L2.
+__device__ __forceinline__ int xcd_tile(int bid, int n_tiles) {
+  return (n_tiles & 7) == 0 ? (bid & 7) * (n_tiles >> 3) + (bid >> 3) : bid;
+}
+
+// Tile t -> (n-block, m-block). Tiles come in groups of kGroupM m-blocks: within a group
+// the m-block varies fastest, so the tiles running at the same time on one XCD share both
+// X row blocks (kGroupM of them) and weight slices (one per kGroupM tiles) in its L2.
+// With at most kGroupM m-blocks this is the plain n-block-major order.
+constexpr int kGroupM = 8;
+__device__ __forceinline__ void tile_coords(int t, int n_mtiles, int n_tiles, int& nt, int& mt) {
+  const int n_ntiles = n_tiles / n_mtiles;
+  const int per_group = kGroupM * n_ntiles;
+  const int grp = t / per_group, r = t - grp * per_group;
+  const int gm = min(kGroupM, n_mtiles - grp * kGroupM);  // m-blocks in this group
+  nt = r / gm;
+  mt = grp * kGroupM + (r - nt * gm);
+}
+
+// Waits until at most n (clamped to 0 .. STAGES - 1) steps of kLoads loads each are in flight.
+template <int STAGES, int kLoads>
+__device__ __forceinline__ void pg_wait_steps(int n) {
+  static_assert(STAGES >= 2 && STAGES <= 8, "stages");
+  switch (n <= 0 ? 0 : (n >= STAGES - 1 ? STAGES - 1 : n)) {
+    case 0: pg_wait<0>(); break;
+    case 1: pg_wait<kLoads>(); break;
+    case 2: pg_wait<(STAGES > 2 ? 2 : 0) * kLoads>(); break;
+    case 3: pg_wait<(STAGES > 3 ? 3 : 0) * kLoads>(); break;
+    case 4: pg_wait<(STAGES > 4 ? 4 : 0) * kLoads>(); break;
+    case 5: pg_wait<(STAGES > 5 ? 5 : 0) * kLoads>(); break;
+    case 6: pg_wait<(STAGES > 6 ? 6 : 0) * kLoads>(); break;
+    default: pg_wait<(STAGES > 7 ? 7 : 0) * kLoads>(); break;
+  }
+}
+// Workgroup barrier without the compiler's memory fence; each side waits for exactly the
+// memory operations it must (the fence would drain every outstanding global load).
+__device__ __forceinline__ void pg_barrier_lds() {
+  asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+}
+__device__ __forceinline__ void pg_barrier() { asm volatile("s_barrier" ::: "memory"); }
+
+// ---------------------------------------------------------------------------------------
+// Shape of one pair_pc_kernel instance. Consumer (wm, wn) of the WM x (4 / WM) consumers owns
+// rows BM/WM * wm .. + BM/WM and pairs kWP * wn .. + kWP (low and high columns).
+template <int BM, int BP, int NPROD, int STAGES, int WM>
+struct PcShape {
+  static constexpr int kConsumers = 4, kWN = kConsumers / WM;
+  static constexpr int kThreads = (kConsumers + NPROD) * 64;
+  static constexpr int kWP = BP / kWN, kPB = kWP / 16, kRB = BM / (16 * WM);
+  static constexpr int kABytes = BM * 128;                 // X tile of one step
+  static constexpr int kStageBytes = kABytes + 2 * BP * 128;  // + W tile (low, high columns)
+  static constexpr int kLoads = kStageBytes / 1024 / NPROD;   // 1 KB loads per producer/step
+  // Epilogue staging in the stage memory once the reduction is done: the fp32 sums as rows
+  // of [BP low | BP high] columns (row stride padded by 4 floats), then the rows' places.
+  static constexpr int kEpStride = 2 * BP + 4;
+  static constexpr int kEpMetaOff = BM * kEpStride * 4;
+  static_assert(kPB >= 1 && kRB >= 1 && kPB * 16 * kWN == BP && kRB * 16 * WM == BM, "tile shape");
+  static_assert(kLoads * NPROD * 1024 == kStageBytes, "producer split");
+  static_assert((STAGES - 1) * kLoads < 64, "vmcnt range");
+  static_assert(STAGES * kStageBytes <= 160 * 1024, "LDS");
+  static_assert(kEpMetaOff + BM * 8 <= STAGES * kStageBytes, "epilogue staging");
+  static_assert(BM <= kThreads, "row destinations");
+};
+
+template <class Ep, int BM, int BP, int NPROD, int STAGES, int WM>
+__global__ __launch_bounds__((4 + NPROD) * 64, 1) void pair_pc_kernel(PairGemmTiles t, Ep ep) {
+  using Sh = PcShape<BM, BP, NPROD, STAGES, WM>;
+  constexpr int kWP = Sh::kWP, kPB = Sh::kPB, kRB = Sh::kRB, kLoads = Sh::kLoads;
+  constexpr int kStageBytes = Sh::kStageBytes, kEpStride = Sh::kEpStride;
+  constexpr int kThreads = Sh::kThreads, kConsumers = Sh::kConsumers;
+  __shared__ __align__(1024) uint8_t smem[STAGES * kStageBytes];
+
+  const int tid = threadIdx.x;
+  int nt, mt;
+  const int n_tiles = t.n_mtiles * t.n_ntiles;
+  tile_coords(xcd_tile(blockIdx.x, n_tiles), t.n_mtiles, n_tiles, nt, mt);
+  const int64_t m0 = int64_t(mt) * BM;
+  const int D = t.k;
+  // The wavefront index is uniform; readfirstlane makes the role test a scalar branch, so a
+  // wavefront executes only its own role's barriers (both roles execute 3 + nk of them).
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
+  const bool producer = wave >= kConsumers;
+  const int nk = D / kPgKT;
+
+  // Places of tile rows 0 .. BM - 1 (threads 0 .. BM - 1), found now and staged in LDS for the
+  // epilogue once the stage memory is free.
+  typename Ep::Row my_row = {};
+  static_assert(sizeof(my_row) == 8, "row places");
+  if (tid < BM) my_row = ep.row(m0 + tid);
+
+  if (producer) {
+    const int pw = wave - kConsumers;
+    // Load i of producer pw fills LDS bytes [1024 q, 1024 q + 1024) of the step's tile
+    // (q = NPROD i + pw, an 8-row block): lane -> row 8 q + lane / 8, LDS chunk lane % 8,
+    // which holds the row's logical chunk (lane % 8) ^ ((row >> 1) & 7) (the LDS tile
+    // layout). Tile rows past n_rows re-read row n_rows - 1 (never stored). The blocks are
+    // dealt round-robin, so every producer requests both X and weight rows: with the X rows
+    // on some producers and the weights on the others, the 40-row projection took 2% longer.
+    const uint16_t* src[kLoads];
+    int dst_off[kLoads];
+#pragma unroll
+    for (int i = 0; i < kLoads; ++i) {
+      const int q = NPROD * i + pw;
+      const int row = 8 * q + (lane >> 3);
+      const int c = (lane & 7) ^ ((row >> 1) & 7);
+      if (row < BM) {
+        src[i] = t.x + min(m0 + row, t.n_rows - 1) * D + 8 * c;
+      } else {
+        const int wr = row - BM, hlf = wr / BP;
+        src[i] = ep.wrow(BP * nt + (wr - hlf * BP), hlf) + 8 * c;
+      }
+      dst_off[i] = 1024 * q;
+    }
+    // With one row block every workgroup reads weights of its own, and starts its walk over the
+    // reduction at its own place: when all of them read the same 128 bytes of their rows (a
+    // power of two apart) at a time, the reads crowd on few HBM channels. Cold weights: gate and
+    // up at 64 rows (201 MB) 46.8 -> 37.1 us, the 40-row projection (101 MB) 24.1 -> 22.3 us,
+    // 128 rows of gate and up 50.9 -> 45.3 us. Row blocks that share weights keep in step (a
+    // start per tile or per XCD gained nothing at 512 to 6842 rows).
+    const int rot = t.n_mtiles == 1 ? static_cast<int>(int64_t(nt) * nk / t.n_ntiles) : 0;
+    // Requests step kt (< nk) into `stage`. No step past the end is requested: the tail of the
+    // loop waits for fewer steps instead (re-reading the last step there, to keep one wait
+    // count, cost 1.3% at 512 rows).
+    auto issue = [&](int kt, int stage) {
+      const int k0 = (kt + rot < nk ? kt + rot : kt + rot - nk) * kPgKT;
+      uint8_t* st = smem + stage * kStageBytes;
+#pragma unroll
+      for (int i = 0; i < kLoads; ++i)
+        __builtin_amdgcn_global_load_lds((PgGlb)(src[i] + k0), (PgLds)(st + dst_off[i]), 16,
+                                         0, 0);
+    };
+    const int first = min(STAGES, nk);  // steps requested before the loop
+#pragma unroll
+    for (int s = 0; s < STAGES; ++s)
+      if (s < first) issue(s, s);
+    pg_wait_steps<STAGES, kLoads>(first - 1);  // step 0 landed
+    pg_barrier();
+    int stage = 0;
+    int kt = 0;
+    for (; kt + STAGES < nk; ++kt) {
+      // step kt + 1 landed (steps kt + 2 .. kt + STAGES - 1 may still be in flight)
+      pg_wait<(STAGES - 2) * kLoads>();
+      pg_barrier();
+      issue(kt + STAGES, stage);  // this stage's last reads came before the barrier
+      stage = stage == STAGES - 1 ? 0 : stage + 1;
+    }
+    // the last steps request nothing: step kt + 1 landed, steps kt + 2 .. nk - 1 in flight
+    for (; kt < nk; ++kt) {
+      pg_wait_steps<STAGES, kLoads>(nk - 2 - kt);
+      pg_barrier();
+    }
+    pg_wait<0>();  // no load may still be writing LDS when the stages are reused
+    pg_barrier();   // -> the consumers may overwrite the stages
+    pg_barrier();   // <- the accumulators and destinations are staged
+  } else {
+    const int wm = wave / Sh::kWN, wn = wave % Sh::kWN;
+    const int l16 = lane & 15, g4 = lane >> 4;
+    const int sw = (l16 >> 1) & 7;
+    struct Frag {
+      u32x4 a[kRB];
+      u32x4 b[2][kPB];
+    };
+    // MFMA operands of half-step ss of the step in `stage`: lane (l16, g4) takes logical
+    // chunk 4 ss + g4 of its row.
+    auto read_frag = [&](Frag& f, int stage, int ss) {
+      const u32x4* st = reinterpret_cast<const u32x4*>(smem + stage * kStageBytes);
+      const int c = (4 * ss + g4) ^ sw;
+#pragma unroll
+      for (int rb = 0; rb < kRB; ++rb) f.a[rb] = st[((BM / WM) * wm + 16 * rb + l16) * 8 + c];
+#pragma unroll
+      for (int h = 0; h < 2; ++h)
+#pragma unroll
+        for (int pb = 0; pb < kPB; ++pb)
+          f.b[h][pb] = st[Sh::kABytes / 16 + (BP * h + kWP * wn + 16 * pb + l16) * 8 + c];
+    };
+    f32x4 acc[kRB][2][kPB];
+#pragma unroll
+    for (int rb = 0; rb < kRB; ++rb)
+#pragma unroll
+      for (int h = 0; h < 2; ++h)
+#pragma unroll
+        for (int pb = 0; pb < kPB; ++pb) acc[rb][h][pb] = f32x4{0.f, 0.f, 0.f, 0.f};
+    auto mma = [&](const Frag& f) {
+#pragma unroll
+      for (int rb = 0; rb < kRB; ++rb)
+#pragma unroll
+        for (int h = 0; h < 2; ++h)
+#pragma unroll
+          for (int pb = 0; pb < kPB; ++pb)
+            acc[rb][h][pb] = mfma16(as_bf16x8(f.a[rb]), as_bf16x8(f.b[h][pb]), acc[rb][h][pb]);
+    };
+    // the next half-step's LDS reads spread between this half-step's MFMAs
+    constexpr int kReads = kRB + 2 * kPB, kMfma = 2 * kRB * kPB;
+    constexpr int kEvery = kMfma / kReads;  // MFMAs after each read
+    auto interleave = [&]() {
+      if constexpr (kEvery == 0) return;  // fewer MFMAs than reads: the compiler's order
+#pragma unroll
+      for (int i = 0; i < kReads; ++i) {
+        __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
+        __builtin_amdgcn_sched_group_barrier(0x008, kEvery, 0);
+      }
+      if constexpr (kMfma > kEvery * kReads)
+        __builtin_amdgcn_sched_group_barrier(0x008, kMfma - kEvery * kReads, 0);
+    };
+
+    Frag f0, f1;
+    pg_barrier_lds();  // step 0 landed
+    read_frag(f0, 0, 0);
+    int stage = 0;
+    for (int kt = 0; kt < nk; ++kt) {
+      const int next = stage == STAGES - 1 ? 0 : stage + 1;
+      read_frag(f1, stage, 1);
+      mma(f0);
+      interleave();
+      __builtin_amdgcn_sched_barrier(0);
+      pg_barrier_lds();  // step kt + 1 landed; this wave's reads of step kt done
+      __builtin_amdgcn_sched_barrier(0);
+      read_frag(f0, next, 0);
+      mma(f1);
+      interleave();
+      __builtin_amdgcn_sched_barrier(0);
+      stage = next;
+    }
+
+    // Stage the accumulators as fp32 rows in LDS: acc[rb][h][pb][i] is row
+    // BM/WM wm + 16 rb + 4 g4 + i, local pair kWP wn + 16 pb + l16, low (h = 0) or high.
+    pg_barrier_lds();  // every LDS read done, every producer load landed
+    float* staged = reinterpret_cast<float*>(smem);
+#pragma unroll
+    for (int rb = 0; rb < kRB; ++rb)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        float* row = staged + ((BM / WM) * wm + 16 * rb + 4 * g4 + i) * kEpStride + kWP * wn + l16;
+#pragma unroll
+        for (int h = 0; h < 2; ++h)
+#pragma unroll
+          for (int pb = 0; pb < kPB; ++pb) row[BP * h + 16 * pb] = acc[rb][h][pb][i];
+      }
+    if (tid < BM) reinterpret_cast<typename Ep::Row*>(smem + Sh::kEpMetaOff)[tid] = my_row;
+    pg_barrier_lds();
+  }
+
+  // Every thread stores groups of 8 pairs of one row (16-byte stores): all the reads of its
+  // groups first, then the stores.
+  const float* staged = reinterpret_cast<const float*>(smem);
+  const auto* meta = reinterpret_cast<const typename Ep::Row*>(smem + Sh::kEpMetaOff);
+  constexpr int kGroups = BP / 8, kItems = BM * kGroups;
+  constexpr int kPer = (kItems + kThreads - 1) / kThreads;
+  typename Ep::Group grp[kPer];
+#pragma unroll
+  for (int j = 0; j < kPer; ++j) {
+    const int it = min(tid + kThreads * j, kItems - 1);
+    const int row = it / kGroups, g = it - kGroups * row;
+    const bool mine = kItems % kThreads == 0 || tid + kThreads * j < kItems;
+    grp[j].load(ep, meta[row], m0 + row, BP * nt + 8 * g, staged + row * kEpStride + 8 * g, BP, mine);
+  }
+#pragma unroll
+  for (int j = 0; j < kPer; ++j) grp[j].store(ep);
+}
+
+// ---------------------------------------------------------------------------------------
+// 256-row tiles
+
 // Tile t -> (n-block, m-block): groups of up to kPgGroupM m-blocks, the m-block fastest within
 // a group, so that the tiles of one XCD share x rows and weight rows in its L2.
 // At 27 m-blocks (6842 rows): groups of at most 4 / 6 / 8 take 540 / 543 / 567 us.
@@ -95,15 +377,10 @@ __device__ __forceinline__ void pg_tile(const PairGemmTiles& t, int i, int& nt, 
   mt = grp * gm + (r - nt * in_grp);
 }
 
-// Epilogue `Ep`: wrow(p, hi) is the first element of pair p's low or high weight row; row(r) ->
-// Ep::Row (8 bytes) says where output row r goes (also for r past n_rows: nowhere);
-// store(row, r, p, lo, hi) takes the sums of pairs p .. p + 7 (p a multiple of 8) of row r from
-// LDS.
 template <class Ep>
 __global__ __launch_bounds__(kPgThreads, 1) void pair_gemm_kernel(PairGemmTiles t, Ep ep) {
   constexpr int kRB = 4, kPB = 3, kWP = kPgBP / 2;
   __shared__ __align__(1024) uint8_t smem[kPgLds];
-  typedef __attribute__((address_space(3))) void* lds_p;
 
   const int tid = threadIdx.x;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
@@ -140,7 +417,7 @@ __global__ __launch_bounds__(kPgThreads, 1) void pair_gemm_kernel(PairGemmTiles 
     const int hi = row / kPgBP;
     bsrc[l] = ep.wrow(kPgBP * nt + (row - hi * kPgBP), hi) + 8 * c;
   }
-  const uint32_t lds0 = static_cast<uint32_t>(reinterpret_cast<size_t>((lds_p)smem));
+  const uint32_t lds0 = static_cast<uint32_t>(reinterpret_cast<size_t>((PgLds)smem));
   const uint32_t a_lds = __builtin_amdgcn_readfirstlane(lds0 + 1024 * wave);
   const uint32_t b_lds = __builtin_amdgcn_readfirstlane(lds0 + kPgBOff + 1024 * wave);
   auto load_a = [&](int stage, int l) {
@@ -266,9 +543,43 @@ __global__ __launch_bounds__(kPgThreads, 1) void pair_gemm_kernel(PairGemmTiles 
       const int row = it / kGroups, g = it - kGroups * row;
       const float* src = epm + row * kPgEpStride + 8 * g;
       const int mrow = kPgEpRows * half + row;
-      ep.store(meta[mrow], m0 + mrow, kPgBP * nt + 8 * g, src, src + kPgBP);
+      typename Ep::Group grp;
+      grp.load(ep, meta[mrow], m0 + mrow, kPgBP * nt + 8 * g, src, kPgBP, true);
+      grp.store(ep);
     }
   }
+}
+
+// ---------------------------------------------------------------------------------------
+// Launch
+
+// Compute units of the current device (cached per device).
+inline int pg_device_cus() {
+  static std::atomic<int> cache[64];
+  int dev = 0;
+  if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) return 256;
+  int n = cache[dev].load(std::memory_order_relaxed);
+  if (n == 0) {
+    if (hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess ||
+        n <= 0)
+      n = 256;
+    cache[dev].store(n, std::memory_order_relaxed);
+  }
+  return n;
+}
+
+// `kernel` of BM-row, BP-pair tiles over n_rows rows and n_pairs pairs (a multiple of BP).
+template <class Ep>
+hipError_t pair_launch(void (*kernel)(PairGemmTiles, Ep), int bm, int bp, int threads,
+                       const uint16_t* x, int64_t n_rows, int64_t k, int64_t n_pairs, const Ep& ep,
+                       hipStream_t stream) {
+  const int64_t n_mtiles = (n_rows + bm - 1) / bm, n_ntiles = n_pairs / bp;
+  if (n_mtiles * n_ntiles >= (int64_t(1) << 31)) return hipErrorInvalidValue;
+  const PairGemmTiles t = {x, n_rows, static_cast<int>(k), static_cast<int>(n_mtiles),
+                           static_cast<int>(n_ntiles)};
+  hipLaunchKernelGGL(kernel, dim3(static_cast<unsigned>(n_mtiles * n_ntiles)), dim3(threads), 0,
+                     stream, t, ep);
+  return hipGetLastError();
 }
 
 }  // namespace fdl

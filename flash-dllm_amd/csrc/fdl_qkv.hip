@@ -41,7 +41,6 @@ namespace {
 
 constexpr int kHeadDim = 128;
 constexpr int kHalf = 64;
-constexpr int kKT = 64;  // reduction step, bf16 elements (8 chunks of 16 B per row)
 constexpr int kDAlign = 256;  // d_model must be a multiple of this
 
 struct QkvArgs {
@@ -59,36 +58,9 @@ struct QkvArgs {
   int64_t n_kv_rows;
   int d_model;
   int n_heads;
-  int n_mtiles;
-  int n_tiles;
   int kv_packed;
   int rope_half;  // sin/cos rows repeat their first half: read only that half
 };
-
-// LDS tile layout: chunk c (16 B) of tile row r is stored at chunk c ^ ((r >> 1) & 7) of
-// that row: two 128-byte rows share one 256-byte bank line, so 16 consecutive rows read at
-// the same logical chunk land on 16 distinct 4-bank groups.
-
-// Workgroup i runs on XCD i % 8. Renumber so that each XCD gets a contiguous run of tiles
-// (tiles are numbered n-block-major): the m-tiles that share one weight slice then run on
-// one XCD and share its L2.
-__device__ __forceinline__ int xcd_tile(int bid, int n_tiles) {
-  return (n_tiles & 7) == 0 ? (bid & 7) * (n_tiles >> 3) + (bid >> 3) : bid;
-}
-
-// Tile t -> (n-block, m-block). Tiles come in groups of kGroupM m-blocks: within a group
-// the m-block varies fastest, so the tiles running at the same time on one XCD share both
-// X row blocks (kGroupM of them) and weight slices (one per kGroupM tiles) in its L2.
-// With at most kGroupM m-blocks this is the plain n-block-major order.
-constexpr int kGroupM = 8;
-__device__ __forceinline__ void tile_coords(int t, int n_mtiles, int n_tiles, int& nt, int& mt) {
-  const int n_ntiles = n_tiles / n_mtiles;
-  const int per_group = kGroupM * n_ntiles;
-  const int grp = t / per_group, r = t - grp * per_group;
-  const int gm = min(kGroupM, n_mtiles - grp * kGroupM);  // m-blocks in this group
-  nt = r / gm;
-  mt = grp * kGroupM + (r - nt * gm);
-}
 
 // Destinations of row r: dq = Q row, dkv = K/V row (cache slot, or the packed row), rope =
 // sin/cos row. A row past n_rows, or with an out-of-range slot or rope row, gets -1 in all
@@ -179,264 +151,13 @@ struct EpGroup {
   }
 };
 
-typedef __attribute__((address_space(3))) void* lds_ptr;
-typedef __attribute__((address_space(1))) void* glb_ptr;
-
-template <int N>
-__device__ __forceinline__ void wait_vmcnt() {
-  static_assert(N >= 0 && N < 64, "vmcnt");
-  asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory");
-}
-// Waits until at most n (clamped to 0 .. STAGES - 1) steps of kLoads loads each are in flight.
-template <int STAGES, int kLoads>
-__device__ __forceinline__ void wait_steps(int n) {
-  static_assert(STAGES >= 2 && STAGES <= 8, "stages");
-  switch (n <= 0 ? 0 : (n >= STAGES - 1 ? STAGES - 1 : n)) {
-    case 0: wait_vmcnt<0>(); break;
-    case 1: wait_vmcnt<kLoads>(); break;
-    case 2: wait_vmcnt<(STAGES > 2 ? 2 : 0) * kLoads>(); break;
-    case 3: wait_vmcnt<(STAGES > 3 ? 3 : 0) * kLoads>(); break;
-    case 4: wait_vmcnt<(STAGES > 4 ? 4 : 0) * kLoads>(); break;
-    case 5: wait_vmcnt<(STAGES > 5 ? 5 : 0) * kLoads>(); break;
-    case 6: wait_vmcnt<(STAGES > 6 ? 6 : 0) * kLoads>(); break;
-    default: wait_vmcnt<(STAGES > 7 ? 7 : 0) * kLoads>(); break;
-  }
-}
-// Workgroup barrier without the compiler's memory fence; each side waits for exactly the
-// memory operations it must (the fence would drain every outstanding global load).
-__device__ __forceinline__ void barrier_lds_drained() {
-  asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
-}
-__device__ __forceinline__ void barrier_only() { asm volatile("s_barrier" ::: "memory"); }
-
-// ---------------------------------------------------------------------------------------
-// Shape of one qkv_pc_kernel instance. Consumer (wm, wn), wm, wn < 2, owns rows
-// BM/2 * wm .. + BM/2 and pairs BP/2 * wn .. + BP/2 (low and high columns).
-template <int BM, int BP, int NPROD, int STAGES>
-struct PcShape {
-  static constexpr int kConsumers = 4;
-  static constexpr int kThreads = (kConsumers + NPROD) * 64;
-  static constexpr int kWP = BP / 2, kPB = kWP / 16, kRB = BM / 32;
-  static constexpr int kABytes = BM * 128;                 // X tile of one step
-  static constexpr int kStageBytes = kABytes + 2 * BP * 128;  // + W tile (low, high columns)
-  static constexpr int kLoads = kStageBytes / 1024 / NPROD;   // 1 KB loads per producer/step
-  // Epilogue staging in the stage memory once the reduction is done: the fp32 sums as rows
-  // of [BP low | BP high] columns (row stride padded by 4 floats), then the rows'
-  // destinations (Q row, K/V row, sin/cos row).
-  static constexpr int kEpStride = 2 * BP + 4;
-  static constexpr int kEpMetaOff = BM * kEpStride * 4;
-  static_assert(kPB >= 1 && kRB >= 1 && kPB * 16 == kWP && kRB * 32 == BM, "tile shape");
-  static_assert(kLoads * NPROD * 1024 == kStageBytes, "producer split");
-  static_assert((STAGES - 1) * kLoads < 64, "vmcnt range");
-  static_assert(STAGES * kStageBytes <= 160 * 1024, "LDS");
-  static_assert(kEpMetaOff + 3 * BM * 8 <= STAGES * kStageBytes, "epilogue staging");
-  static_assert(BM <= kThreads, "row destinations");
-};
-
-template <int BM, int BP, int NPROD, int STAGES>
-__global__ __launch_bounds__((4 + NPROD) * 64, 1) void qkv_pc_kernel(QkvArgs a) {
-  using Sh = PcShape<BM, BP, NPROD, STAGES>;
-  constexpr int kWP = Sh::kWP, kPB = Sh::kPB, kRB = Sh::kRB, kLoads = Sh::kLoads;
-  constexpr int kStageBytes = Sh::kStageBytes, kEpStride = Sh::kEpStride;
-  constexpr int kThreads = Sh::kThreads, kConsumers = Sh::kConsumers;
-  __shared__ __align__(1024) uint8_t smem[STAGES * kStageBytes];
-
-  const int tid = threadIdx.x;
-  int nt, mt;
-  tile_coords(xcd_tile(blockIdx.x, a.n_tiles), a.n_mtiles, a.n_tiles, nt, mt);
-  const int64_t m0 = int64_t(mt) * BM;
-  const int D = a.d_model;
-  const int pairs_per_mat = a.n_heads * kHalf;
-  // The wavefront index is uniform; readfirstlane makes the role test a scalar branch, so a
-  // wavefront executes only its own role's barriers (both roles execute 3 + nk of them).
-  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
-  const bool producer = wave >= kConsumers;
-  const int nk = D / kKT;
-
-  // Destinations of tile rows 0 .. BM - 1 (threads 0 .. BM - 1), read now and staged in LDS
-  // for the epilogue once the stage memory is free.
-  int64_t my_dq = -1, my_dkv = -1, my_rope = -1;
-  if (tid < BM) row_dest(a, m0 + tid, my_dq, my_dkv, my_rope);
-
-  if (producer) {
-    const int pw = wave - kConsumers;
-    // Load i of producer pw fills LDS bytes [1024 q, 1024 q + 1024) of the step's tile
-    // (q = NPROD i + pw, an 8-row block): lane -> row 8 q + lane / 8, LDS chunk lane % 8,
-    // which holds the row's logical chunk (lane % 8) ^ ((row >> 1) & 7) (the LDS tile
-    // layout). Tile rows past n_rows re-read row n_rows - 1 (never stored). The blocks are
-    // dealt round-robin, so every producer requests both X and weight rows: with the X rows
-    // on some producers and the weights on the others, the 40-row projection took 2% longer.
-    const uint16_t* src[kLoads];
-    int dst_off[kLoads];
-#pragma unroll
-    for (int i = 0; i < kLoads; ++i) {
-      const int q = NPROD * i + pw;
-      const int row = 8 * q + (lane >> 3);
-      const int c = (lane & 7) ^ ((row >> 1) & 7);
-      if (row < BM) {
-        src[i] = a.x + min(m0 + row, a.n_rows - 1) * D + 8 * c;
-      } else {
-        const int wr = row - BM, hlf = wr / BP;
-        const int p = BP * nt + (wr - hlf * BP);
-        const int mat = p / pairs_per_mat, rem = p - mat * pairs_per_mat;
-        src[i] = a.w[mat] + int64_t((rem >> 6) * kHeadDim + (rem & 63) + kHalf * hlf) * D +
-                 8 * c;
-      }
-      dst_off[i] = 1024 * q;
-    }
-    // Requests step kt (< nk) into `stage`. No step past the end is requested: the tail of the
-    // loop waits for fewer steps instead (re-reading the last step there, to keep one wait
-    // count, cost 1.3% at 512 rows).
-    auto issue = [&](int kt, int stage) {
-      const int k0 = kt * kKT;
-      uint8_t* st = smem + stage * kStageBytes;
-#pragma unroll
-      for (int i = 0; i < kLoads; ++i)
-        __builtin_amdgcn_global_load_lds((glb_ptr)(src[i] + k0), (lds_ptr)(st + dst_off[i]), 16,
-                                         0, 0);
-    };
-    const int first = min(STAGES, nk);  // steps requested before the loop
-#pragma unroll
-    for (int s = 0; s < STAGES; ++s)
-      if (s < first) issue(s, s);
-    wait_steps<STAGES, kLoads>(first - 1);  // step 0 landed
-    barrier_only();
-    int stage = 0;
-    int kt = 0;
-    for (; kt + STAGES < nk; ++kt) {
-      // step kt + 1 landed (steps kt + 2 .. kt + STAGES - 1 may still be in flight)
-      wait_vmcnt<(STAGES - 2) * kLoads>();
-      barrier_only();
-      issue(kt + STAGES, stage);  // this stage's last reads came before the barrier
-      stage = stage == STAGES - 1 ? 0 : stage + 1;
-    }
-    // the last steps request nothing: step kt + 1 landed, steps kt + 2 .. nk - 1 in flight
-    for (; kt < nk; ++kt) {
-      wait_steps<STAGES, kLoads>(nk - 2 - kt);
-      barrier_only();
-    }
-    wait_vmcnt<0>();  // no load may still be writing LDS when the stages are reused
-    barrier_only();   // -> the consumers may overwrite the stages
-    barrier_only();   // <- the accumulators and destinations are staged
-  } else {
-    const int wm = wave >> 1, wn = wave & 1;  // rows BM/2 wm .., pairs BP/2 wn ..
-    const int l16 = lane & 15, g4 = lane >> 4;
-    const int sw = (l16 >> 1) & 7;
-    struct Frag {
-      u32x4 a[kRB];
-      u32x4 b[2][kPB];
-    };
-    // MFMA operands of half-step ss of the step in `stage`: lane (l16, g4) takes logical
-    // chunk 4 ss + g4 of its row.
-    auto read_frag = [&](Frag& f, int stage, int ss) {
-      const u32x4* st = reinterpret_cast<const u32x4*>(smem + stage * kStageBytes);
-      const int c = (4 * ss + g4) ^ sw;
-#pragma unroll
-      for (int rb = 0; rb < kRB; ++rb) f.a[rb] = st[((BM / 2) * wm + 16 * rb + l16) * 8 + c];
-#pragma unroll
-      for (int h = 0; h < 2; ++h)
-#pragma unroll
-        for (int pb = 0; pb < kPB; ++pb)
-          f.b[h][pb] = st[Sh::kABytes / 16 + (BP * h + kWP * wn + 16 * pb + l16) * 8 + c];
-    };
-    f32x4 acc[kRB][2][kPB];
-#pragma unroll
-    for (int rb = 0; rb < kRB; ++rb)
-#pragma unroll
-      for (int h = 0; h < 2; ++h)
-#pragma unroll
-        for (int pb = 0; pb < kPB; ++pb) acc[rb][h][pb] = f32x4{0.f, 0.f, 0.f, 0.f};
-    auto mma = [&](const Frag& f) {
-#pragma unroll
-      for (int rb = 0; rb < kRB; ++rb)
-#pragma unroll
-        for (int h = 0; h < 2; ++h)
-#pragma unroll
-          for (int pb = 0; pb < kPB; ++pb)
-            acc[rb][h][pb] = mfma16(as_bf16x8(f.a[rb]), as_bf16x8(f.b[h][pb]), acc[rb][h][pb]);
-    };
-    // the next half-step's LDS reads spread between this half-step's MFMAs
-    constexpr int kReads = kRB + 2 * kPB, kMfma = 2 * kRB * kPB;
-    constexpr int kEvery = kMfma / kReads;  // MFMAs after each read
-    static_assert(kEvery >= 1, "interleave");
-    auto interleave = [&]() {
-#pragma unroll
-      for (int i = 0; i < kReads; ++i) {
-        __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
-        __builtin_amdgcn_sched_group_barrier(0x008, kEvery, 0);
-      }
-      if constexpr (kMfma > kEvery * kReads)
-        __builtin_amdgcn_sched_group_barrier(0x008, kMfma - kEvery * kReads, 0);
-    };
-
-    Frag f0, f1;
-    barrier_lds_drained();  // step 0 landed
-    read_frag(f0, 0, 0);
-    int stage = 0;
-    for (int kt = 0; kt < nk; ++kt) {
-      const int next = stage == STAGES - 1 ? 0 : stage + 1;
-      read_frag(f1, stage, 1);
-      mma(f0);
-      interleave();
-      __builtin_amdgcn_sched_barrier(0);
-      barrier_lds_drained();  // step kt + 1 landed; this wave's reads of step kt done
-      __builtin_amdgcn_sched_barrier(0);
-      read_frag(f0, next, 0);
-      mma(f1);
-      interleave();
-      __builtin_amdgcn_sched_barrier(0);
-      stage = next;
-    }
-
-    // Stage the accumulators as fp32 rows in LDS: acc[rb][h][pb][i] is row
-    // BM/2 wm + 16 rb + 4 g4 + i, local pair BP/2 wn + 16 pb + l16, low (h = 0) or high.
-    barrier_lds_drained();  // every LDS read done, every producer load landed
-    float* ep = reinterpret_cast<float*>(smem);
-#pragma unroll
-    for (int rb = 0; rb < kRB; ++rb)
-#pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        float* row = ep + ((BM / 2) * wm + 16 * rb + 4 * g4 + i) * kEpStride + kWP * wn + l16;
-#pragma unroll
-        for (int h = 0; h < 2; ++h)
-#pragma unroll
-          for (int pb = 0; pb < kPB; ++pb) row[BP * h + 16 * pb] = acc[rb][h][pb][i];
-      }
-    if (tid < BM) {
-      int64_t* meta = reinterpret_cast<int64_t*>(smem + Sh::kEpMetaOff);
-      meta[tid] = my_dq;
-      meta[BM + tid] = my_dkv;
-      meta[2 * BM + tid] = my_rope;
-    }
-    barrier_lds_drained();
-  }
-
-  // Every thread rotates and stores groups of 8 pairs of one row (16-byte stores): all the
-  // LDS and sin/cos reads of its groups first, then the stores.
-  const float* ep = reinterpret_cast<const float*>(smem);
-  const int64_t* meta = reinterpret_cast<const int64_t*>(smem + Sh::kEpMetaOff);
-  constexpr int kGroups = BP / 8, kItems = BM * kGroups;
-  constexpr int kPer = (kItems + kThreads - 1) / kThreads;
-  EpGroup grp[kPer];
-#pragma unroll
-  for (int j = 0; j < kPer; ++j) {
-    const int it = min(tid + kThreads * j, kItems - 1);
-    const int row = it / kGroups, g = it - kGroups * row;
-    const int p0 = BP * nt + 8 * g;
-    const int mat = p0 / pairs_per_mat, rem = p0 - mat * pairs_per_mat;
-    const bool mine = kItems % kThreads == 0 || tid + kThreads * j < kItems;
-    grp[j].load(a, ep + row * kEpStride + 8 * g, BP, mat, rem,
-                mine ? meta[(mat == 0 ? 0 : BM) + row] : -1, meta[2 * BM + row]);
-  }
-#pragma unroll
-  for (int j = 0; j < kPer; ++j) grp[j].store(a);
-}
-
-// Epilogue of the 256-row tiles (fdl_pair_gemm.h).
+// Epilogue of the pair GEMM (fdl_pair_gemm.h).
 struct RopeEp {
   QkvArgs a;
   struct Row {
-    int dkv, rope;  // K/V row, sin/cos row (both below 2^31: the host checks); -1: not stored
+    // K/V row, sin/cos row (both below 2^31: a cache or table row takes at least 512 bytes); -1:
+    // not stored
+    int dkv, rope;
   };
   __device__ __forceinline__ const uint16_t* wrow(int p, int hi) const {
     const int pairs_per_mat = a.n_heads * kHalf;
@@ -448,15 +169,17 @@ struct RopeEp {
     row_dest(a, r, dq, dkv, rope);
     return {static_cast<int>(dkv), static_cast<int>(rope)};
   }
-  __device__ __forceinline__ void store(const Row& d, int64_t r, int p, const float* lo,
-                                        const float* hi) const {
-    const int pairs_per_mat = a.n_heads * kHalf;
-    const int mat = p / pairs_per_mat, rem = p - mat * pairs_per_mat;
+  struct Group {
     EpGroup g;
-    g.load(a, lo, static_cast<int>(hi - lo), mat, rem,
-           d.rope < 0 ? -1 : (mat == 0 ? r : int64_t(d.dkv)), d.rope);
-    g.store(a);
-  }
+    __device__ __forceinline__ void load(const RopeEp& ep, const Row& d, int64_t r, int p,
+                                         const float* lo, int hi_off, bool mine) {
+      const int pairs_per_mat = ep.a.n_heads * kHalf;
+      const int mat = p / pairs_per_mat, rem = p - mat * pairs_per_mat;
+      g.load(ep.a, lo, hi_off, mat, rem,
+             !mine || d.rope < 0 ? -1 : (mat == 0 ? r : int64_t(d.dkv)), d.rope);
+    }
+    __device__ __forceinline__ void store(const RopeEp& ep) { g.store(ep.a); }
+  };
 };
 
 }  // namespace
@@ -465,35 +188,7 @@ struct RopeEp {
 namespace fdl {
 namespace {
 
-// A producer / consumer tile shape.
-struct QkvPlan {
-  void (*kernel)(QkvArgs);
-  int bm;       // rows per tile
-  int bp;       // pairs per tile
-  int threads;  // per workgroup
-};
-
 constexpr int kPcBM = 128, kPcBP = 96;
-
-template <int BM, int BP, int NPROD, int STAGES>
-constexpr QkvPlan pc_plan() {
-  return {qkv_pc_kernel<BM, BP, NPROD, STAGES>, BM, BP, PcShape<BM, BP, NPROD, STAGES>::kThreads};
-}
-
-// Compute units of the current device (cached per device).
-int device_cus() {
-  static std::atomic<int> cache[64];
-  int dev = 0;
-  if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) return 256;
-  int n = cache[dev].load(std::memory_order_relaxed);
-  if (n == 0) {
-    if (hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess ||
-        n <= 0)
-      n = 256;
-    cache[dev].store(n, std::memory_order_relaxed);
-  }
-  return n;
-}
 
 // Rows of a call and the shapes that run them: the first `wide` on 256-row tiles, the next
 // `mid` on 128-row tiles, the rest (at most 128) streaming the weights.
@@ -516,7 +211,7 @@ constexpr int kStreamUs[2] = {17, 21};  // up to 64 rows, up to 128
 constexpr int kStreamRows = 128;
 
 QkvSplit qkv_split(int64_t n_rows, int64_t n_pairs) {
-  const int64_t cus = device_cus();
+  const int64_t cus = pg_device_cus();
   auto rounds = [&](int64_t rows, int bm, int bp) {
     return ((rows + bm - 1) / bm * (n_pairs / bp) + cus - 1) / cus;
   };
@@ -560,28 +255,16 @@ QkvArgs qkv_rows(QkvArgs args, int64_t r0, int64_t n) {
   return args;
 }
 
-hipError_t qkv_launch(const QkvPlan& plan, QkvArgs args, hipStream_t stream) {
-  const int64_t n_pairs = 3 * int64_t(args.n_heads) * kHalf;  // a multiple of every plan's bp
-  const int64_t n_mtiles = (args.n_rows + plan.bm - 1) / plan.bm;
-  const int64_t n_tiles = n_mtiles * (n_pairs / plan.bp);
-  if (n_tiles >= (int64_t(1) << 31)) return hipErrorInvalidValue;
-  args.n_mtiles = static_cast<int>(n_mtiles);
-  args.n_tiles = static_cast<int>(n_tiles);
-  hipLaunchKernelGGL(plan.kernel, dim3(static_cast<unsigned>(n_tiles)), dim3(plan.threads), 0,
-                     stream, args);
-  return hipGetLastError();
+hipError_t qkv_launch(void (*kernel)(PairGemmTiles, RopeEp), int bm, int bp, int threads,
+                      const QkvArgs& args, hipStream_t stream) {
+  return pair_launch(kernel, bm, bp, threads, args.x, args.n_rows, args.d_model,
+                     3 * int64_t(args.n_heads) * kHalf, RopeEp{args}, stream);
 }
 
-hipError_t qkv_launch_wide(const QkvArgs& args, hipStream_t stream) {
-  const int64_t n_pairs = 3 * int64_t(args.n_heads) * kHalf;
-  const int64_t n_mtiles = (args.n_rows + kPgBM - 1) / kPgBM;
-  const int64_t n_tiles = n_mtiles * (n_pairs / kPgBP);
-  if (n_tiles >= (int64_t(1) << 31)) return hipErrorInvalidValue;
-  const PairGemmTiles t = {args.x, args.n_rows, args.d_model, static_cast<int>(n_mtiles),
-                           static_cast<int>(n_pairs / kPgBP)};
-  hipLaunchKernelGGL(pair_gemm_kernel<RopeEp>, dim3(static_cast<unsigned>(n_tiles)),
-                     dim3(kPgThreads), 0, stream, t, RopeEp{args});
-  return hipGetLastError();
+template <int BM, int BP, int NPROD, int STAGES>
+hipError_t qkv_launch_pc(const QkvArgs& args, hipStream_t stream) {
+  return qkv_launch(pair_pc_kernel<RopeEp, BM, BP, NPROD, STAGES, 2>, BM, BP,
+                    PcShape<BM, BP, NPROD, STAGES, 2>::kThreads, args, stream);
 }
 
 }  // namespace
@@ -655,19 +338,20 @@ extern "C" int fdl_qkv_rope_cache(const void* x, const void* wq, const void* wk,
   args.n_kv_rows = n_kv_rows;
   args.d_model = static_cast<int>(d_model);
   args.n_heads = static_cast<int>(n_heads);
-  args.n_mtiles = 0;
-  args.n_tiles = 0;
   args.kv_packed = kv_packed;
   args.rope_half = (flags & FDL_QKV_ROPE_HALVES_EQUAL) ? 1 : 0;
   const hipStream_t st = static_cast<hipStream_t>(stream);
   const QkvSplit split = qkv_split(n_rows, 3 * n_heads * kHalf);
   const int64_t rest = n_rows - split.wide - split.mid;
-  if (split.wide > 0) FDL_HIP_CHECK(qkv_launch_wide(qkv_rows(args, 0, split.wide), st));
+  if (split.wide > 0)
+    FDL_HIP_CHECK(qkv_launch(pair_gemm_kernel<RopeEp>, kPgBM, kPgBP, kPgThreads,
+                             qkv_rows(args, 0, split.wide), st));
   if (split.mid > 0)
-    FDL_HIP_CHECK(qkv_launch(pc_plan<kPcBM, kPcBP, 4, 4>(),
-                             qkv_rows(args, split.wide, split.mid), st));
-  if (rest > 0)
-    FDL_HIP_CHECK(qkv_launch(rest <= 64 ? pc_plan<64, 32, 4, 8>() : pc_plan<128, 32, 4, 6>(),
-                             qkv_rows(args, split.wide + split.mid, rest), st));
+    FDL_HIP_CHECK((qkv_launch_pc<kPcBM, kPcBP, 4, 4>(qkv_rows(args, split.wide, split.mid), st)));
+  if (rest > 0) {
+    const QkvArgs tail = qkv_rows(args, split.wide + split.mid, rest);
+    FDL_HIP_CHECK((rest <= 64 ? qkv_launch_pc<64, 32, 4, 8>(tail, st)
+                              : qkv_launch_pc<128, 32, 4, 6>(tail, st)));
+  }
   return ok();
 }

@@ -150,12 +150,15 @@ def test_qkv_packed_verify_mode(Q):
     (4, 8491),   # a round of 256-row tiles, the rest on 128-row tiles
     (4, 8232),   # a round of 256-row tiles, the rest streamed
     (4, 12304),  # a round of 256-row tiles, one of 128-row tiles, the rest streamed
-    (6, 2801),   # a tile count that is no multiple of 8
+    (6, 2801),   # a round of 128-row tiles, the rest streamed
+    (6, 2816),   # a count of 256-row tiles that is no multiple of 8
 ])
 def test_qkv_rope_cache_many_rows(heads, rows, kv_packed, halves):
-    """Row counts that run 256-row tiles, alone and with a rest on another shape, equal bit for
-    bit to the same rows in calls of at most 500 (128-row tiles: the same products summed in
-    the same order); rows whose slot is out of range stay out of all three outputs."""
+    """Row counts that run 256-row tiles or more than one shape, equal bit for bit to the
+    same rows in calls of at most 500 (128-row tiles: the same products summed in the same
+    order); rows whose slot is out of range stay out of all three outputs. A streamed rest sums
+    in another order: its float32 sums differ by about 1e-6, so its bf16 results by one place at
+    most (2^-7 of the value, or 1e-4 where the rotation cancels)."""
     D = 128 * heads
     gen = torch.Generator().manual_seed(rows)
     n_slots = rows + 99
@@ -180,8 +183,14 @@ def test_qkv_rope_cache_many_rows(heads, rows, kv_packed, halves):
         kv = [t[r:r + 500] for t in parts[1:]] if kv_packed else parts[1:]
         ops.qkv_rope_cache(x[r:r + 500], *w, sin, cos, slot[r:r + 500], parts[0][r:r + 500], *kv,
                            heads, kv_packed=kv_packed)
+    streamed = rows % 128 if rows in (8232, 12304, 2801) else 0
     for name, a, b in zip("QKV", whole, parts):
-        assert torch.equal(a, b), f"{name} differs"
+        same = torch.ones(a.shape[0], dtype=torch.bool)
+        if streamed:
+            at = slot[-streamed:].tolist() if name != "Q" and not kv_packed else range(rows - streamed, rows)
+            same[[i for i in at if 0 <= i < a.shape[0]]] = False
+            torch.testing.assert_close(a[~same].float(), b[~same].float(), rtol=2**-7, atol=1e-4)
+        assert torch.equal(a[same], b[same]), f"{name} differs"
     assert bool((whole[0][7] == POISON).all()) and bool((whole[0][6] != POISON).any())
 
 
