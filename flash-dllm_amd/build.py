@@ -24,8 +24,8 @@ LIB_PATH = PKG_DIR / "libfdl.so"
 ROCM = Path(os.environ.get("ROCM_PATH", "/opt/rocm"))
 ARCH = "gfx950"
 
-HIP_SOURCES = ["fdl_qkv.hip", "fdl_attn.hip", "fdl_rank.hip", "fdl_block.hip", "fdl_head.hip",
-               "fdl_sched.hip"]
+HIP_SOURCES = ["fdl_qkv.hip", "fdl_mlp.hip", "fdl_attn.hip", "fdl_rank.hip", "fdl_block.hip",
+               "fdl_head.hip", "fdl_sched.hip"]
 CXX_SOURCES = ["fdl_host.cpp"]
 
 HIPCC_FLAGS = [
@@ -37,9 +37,9 @@ HIPCC_FLAGS = [
     # keep the compiler from forming packed fp32 ops (v_pk_*_f32)
     "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",
 ]
-# Per-source additions. The QKV kernels keep their MFMA accumulators in VGPRs: with the
+# Per-source additions. The pair GEMM kernels keep their MFMA accumulators in VGPRs: with the
 # accumulators in AGPRs the register allocator shuffles them between loop iterations.
-HIPCC_EXTRA = {"fdl_qkv.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form"]}
+HIPCC_EXTRA = {src: ["-mllvm", "-amdgpu-mfma-vgpr-form"] for src in ("fdl_qkv.hip", "fdl_mlp.hip")}
 CXX_FLAGS = ["-O2", "-std=c++17", "-fPIC", "-Wall", "-Wextra"]
 
 

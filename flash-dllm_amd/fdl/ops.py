@@ -451,6 +451,36 @@ def silu_mul(gate: torch.Tensor, up: torch.Tensor, out: torch.Tensor | None = No
     return out
 
 
+def gate_up_silu_pays(rows: int, width: int, device: torch.device) -> bool:
+    """Whether gate_up_silu is faster than one library product over both weights and silu_mul:
+    while its 128-row tiles fit one round of workgroups (width 12288: up to 256 rows; 64 rows
+    50 -> 37 us, 256 rows 67 -> 61 us; 640 rows 132 -> 158 us)."""
+    return 0 < rows and -(-rows // 128) * (width // 96) <= _cus(device)
+
+
+def gate_up_silu(x: torch.Tensor, w_gate: torch.Tensor, w_up: torch.Tensor,
+                 out_chunks: int = 1) -> torch.Tensor:
+    """bf16(bf16(silu(x w_gate^T)) * (x w_up^T)) with both products rounded to bf16
+    (fdl_gate_up_silu): x [rows, k], weights [width, k] -> [rows, width], or with out_chunks = S
+    > 1 the column chunks [S, rows, width / S]. k a multiple of 128 from 256 on, width a multiple
+    of 96."""
+    dev = x.device
+    _need(x, "x", BF16, 2)
+    _need(w_gate, "w_gate", BF16, 2, dev)
+    _need(w_up, "w_up", BF16, 2, dev)
+    rows, k = x.shape
+    width = w_gate.shape[0]
+    if w_gate.shape[1] != k or w_up.shape != w_gate.shape:
+        raise _lib.FdlError(_lib.FDL_ERR_SHAPE, "w_gate and w_up must both be [width, k]")
+    if out_chunks < 1 or width % out_chunks:
+        raise _lib.FdlError(_lib.FDL_ERR_SHAPE, f"out_chunks {out_chunks} does not divide {width}")
+    out = torch.empty((rows, width) if out_chunks == 1 else (out_chunks, rows, width // out_chunks),
+                      dtype=BF16, device=dev)
+    _lib.call("fdl_gate_up_silu", x.data_ptr(), w_gate.data_ptr(), w_up.data_ptr(), rows, k, width,
+              out_chunks, out.data_ptr(), _stream(x))
+    return out
+
+
 def split_reduce_residual(part: torch.Tensor, residual: torch.Tensor) -> torch.Tensor:
     """residual = bf16(residual + sum_s part[s]) in place (fdl_split_reduce_residual):
     part fp32 [S, rows, cols], residual bf16 [rows, cols]."""

@@ -157,6 +157,16 @@ def _adjacent_gate_up(block) -> torch.Tensor | None:
     return torch.as_strided(wg, (2 * h, d), (d, 1))
 
 
+def _fused_gate_up(x: torch.Tensor, w_gu: torch.Tensor) -> bool:
+    """Whether the gate and up products and the SiLU gate run as one kernel
+    (ops.gate_up_silu): the shapes it takes, at row counts where it is the faster way."""
+    width, k = w_gu.shape[0] // 2, w_gu.shape[1]
+    return (x.dim() == 2 and x.is_cuda and x.is_contiguous() and w_gu.dtype == torch.bfloat16
+            and width % 96 == 0 and k % 128 == 0 and 256 <= k <= 65536
+            and x.data_ptr() % 16 == 0 and w_gu.data_ptr() % 16 == 0
+            and ops.gate_up_silu_pays(x.shape[0], width, x.device))
+
+
 # ff_out (K = mlp width, N = d_model) as a split-K product at up to SPLIT_K_MAX_ROWS rows:
 # at 512 rows its N = 4096 outputs give too few tiles for the CUs; four K-chunks as one
 # batched product with float32 partials, then one pass that adds them and the residual,
@@ -212,18 +222,23 @@ def block_mlp_tail(self, x: torch.Tensor, att: torch.Tensor) -> torch.Tensor:
     w_gu = _adjacent_gate_up(self)
     if w_gu is not None and ck is None and isinstance(self.act, torch.nn.SiLU) \
             and x.dtype == torch.bfloat16:
-        # one GEMM over the concatenated ff_proj / up_proj weights, then SiLU(gate) * up
-        # over the two halves of each output row
+        # one pass over the concatenated ff_proj / up_proj weights, or one GEMM over them, then
+        # SiLU(gate) * up over the two halves of each output row
         h = self.ff_proj.weight.shape[0]
-        gu = F.linear(x, w_gu)
-        ws = _split_k_ff_out(self, gu.shape[0])
-        if ws is not None and og_x.is_contiguous() and og_x.dtype == torch.bfloat16:
-            # SiLU(gate) * up written as the K-chunks [S, rows, K / S]; the batched product's
-            # right operands are contiguous chunks of W^T; partials + residual in one pass
-            xs = ops.silu_mul(gu[:, :h], gu[:, h:], out_chunks=ws.shape[0])
-            part = torch.bmm(xs, ws, out_dtype=torch.float32)
+        ws = _split_k_ff_out(self, x.shape[0])
+        split = ws is not None and og_x.is_contiguous() and og_x.dtype == torch.bfloat16
+        # SiLU(gate) * up written as the K-chunks [S, rows, K / S] of a split-K ff_out
+        chunks = ws.shape[0] if split else 1
+        if _fused_gate_up(x, w_gu):
+            x = ops.gate_up_silu(x, w_gu[:h], w_gu[h:], out_chunks=chunks)
+        else:
+            gu = F.linear(x, w_gu)
+            x = ops.silu_mul(gu[:, :h], gu[:, h:], out_chunks=chunks)
+        if split:
+            # the batched product's right operands are contiguous chunks of W^T; partials +
+            # residual in one pass
+            part = torch.bmm(x, ws, out_dtype=torch.float32)
             return ops.split_reduce_residual(part, og_x).unsqueeze(0)
-        x = ops.silu_mul(gu[:, :h], gu[:, h:])
         return _ff_out_residual(self, x, og_x).unsqueeze(0)
     x, x_up = self.ff_proj(x), self.up_proj(x)
     if ck is None and isinstance(self.act, torch.nn.SiLU) and x.dtype == torch.bfloat16:

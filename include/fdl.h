@@ -291,6 +291,16 @@ int fdl_silu_mul_rows(const void* gate, const void* up, int64_t n_rows, int64_t 
                       int64_t ld, int64_t out_chunks, void* out, void* stream);
 
 /*
+ * Both MLP projections and the SiLU gate (flash_cache_triton.py:628-633) in one pass:
+ *   y[r][c] = bf16(bf16(silu(g)) * u),  g = bf16(x[r] . w_gate[c]),  u = bf16(x[r] . w_up[c])
+ * for x [n_rows][k] and w_gate, w_up [width][k] (bf16, 16-byte aligned; fp32 sums). The output
+ * is cut into out_chunks column chunks as by fdl_silu_mul_rows. k: a multiple of 128 from 256 to
+ * 65536; width: a multiple of 96.
+ */
+int fdl_gate_up_silu(const void* x, const void* w_gate, const void* w_up, int64_t n_rows,
+                     int64_t k, int64_t width, int64_t out_chunks, void* out, void* stream);
+
+/*
  * fdl_split_reduce_residual: the end of a split-K ff_out product with its residual
  * (flash_cache_triton.py:634-636, `x = og_x + ff_out(x)`):
  *   residual_out[i] = bf16(float(residual_out[i]) + (part[0][i] + part[1][i] + ...)),

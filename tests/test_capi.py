@@ -82,6 +82,11 @@ def test_launchers_reject_bad_scalars_without_gpu():
     _expect(lib.FDL_ERR_UNSUPPORTED, "fdl_silu_mul_rows", None, None, 4, 16, 32, 4, None, None)
     _expect(lib.FDL_ERR_NULL, "fdl_silu_mul_rows", None, None, 4, 16, 32, 2, None, None)
     lib.call("fdl_silu_mul_rows", None, None, 0, 16, 32, 1, None, None)  # zero rows: no-op
+    for k, width, chunks in ((128, 96, 1), (320, 96, 1), (256, 128, 1), (256, 96, 5)):
+        _expect(lib.FDL_ERR_UNSUPPORTED, "fdl_gate_up_silu", None, None, None, 4, k, width, chunks,
+                None, None)
+    _expect(lib.FDL_ERR_NULL, "fdl_gate_up_silu", None, None, None, 4, 256, 96, 1, None, None)
+    lib.call("fdl_gate_up_silu", None, None, None, 0, 256, 96, 1, None, None)  # zero rows: no-op
     _expect(lib.FDL_ERR_UNSUPPORTED, "fdl_split_reduce_residual", None, 0, 4, 16, None, None)
     _expect(lib.FDL_ERR_UNSUPPORTED, "fdl_split_reduce_residual", None, 4, 4, 12, None, None)
     _expect(lib.FDL_ERR_NULL, "fdl_split_reduce_residual", None, 4, 4, 16, None, None)

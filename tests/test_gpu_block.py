@@ -159,3 +159,32 @@ def test_block_mlp_tail_split_k_ff_out_matches_single_product():
     torch.cuda.synchronize()
     torch.testing.assert_close(split.squeeze(0).float(), single.squeeze(0).float(), atol=2e-2, rtol=1e-2)
     torch.testing.assert_close(split.squeeze(0).float(), ref, atol=5e-2, rtol=2e-2)
+
+
+@pytest.mark.parametrize("chunks", [1, 4])
+@pytest.mark.parametrize("rows,k,width", [
+    (1, 256, 96), (64, 4096, 12288), (65, 384, 12288), (17, 640, 192),  # weight-streaming tiles
+    (128, 256, 192), (129, 256, 96), (256, 512, 12288),                 # 128-row tiles
+    (257, 256, 12288), (300, 384, 12384), (600, 512, 12288),            # 256-row tiles
+])
+def test_gate_up_silu_matches_unfused(rows, k, width, chunks):
+    """Both products in float32 rounded to bf16, then silu and the product as torch rounds them.
+    A float32 sum of k bf16 products may round to the reference's bf16 neighbour, 2^-8 of the
+    value at most, in g and in u. silu(g) = g sigmoid(g) changes by (1 + |g|) times g's relative
+    change at most (its logarithmic derivative is 1 + g sigmoid(-g)), and two more roundings add
+    2^-9 each on both sides: 2^-8 (1 + |g|) + 2^-8 + 2^-7 of the value, and where g or u
+    crosses zero the sums' own error (1e-5 of unit-scale sums) through the other factor, 1e-3."""
+    gen = torch.Generator().manual_seed(rows + k)
+    x = torch.randn(rows, k, generator=gen).to(torch.bfloat16).to(DEV)
+    wg, wu = ((torch.randn(width, k, generator=gen) * 0.05).to(torch.bfloat16).to(DEV)
+              for _ in range(2))
+    g = (x.float() @ wg.float().t()).to(torch.bfloat16)
+    u = (x.float() @ wu.float().t()).to(torch.bfloat16)
+    ref = torch.nn.functional.silu(g) * u
+    got = ops.gate_up_silu(x, wg, wu, out_chunks=chunks)
+    if chunks > 1:
+        assert got.shape == (chunks, rows, width // chunks)
+        got = got.transpose(0, 1).reshape(rows, width)
+    tol = ref.float().abs() * (2.0**-8 * (2 + g.float().abs()) + 2.0**-7) + 1e-3
+    assert bool(((got.float() - ref.float()).abs() <= tol).all())
+    assert (got != ref).float().mean() < 0.02
