@@ -24,12 +24,17 @@ __device__ __forceinline__ float bf_hi(uint32_t w) {
 }
 __device__ __forceinline__ float round_bf(float f) { return bf2f(f2bf(f)); }
 
-// Row r: chunks of 8 bf16 strided by the workgroup; d % 8 == 0 (checked on the host).
-template <bool kResidual>
+// Row r: chunks of 8 bf16 strided by the workgroup; d % 8 == 0 (checked on the host). The
+// residual is none, bf16 rows, or n_split fp32 partial sums `stride` apart, added in ascending
+// order and rounded to bf16 first.
+enum class Residual { kNone, kRows, kPartials };
+template <Residual kRes>
 __global__ __launch_bounds__(kNormThreads) void rms_norm_kernel(
     const uint16_t* __restrict__ x, const uint16_t* __restrict__ res,
+    const float* __restrict__ part, int n_split, int64_t stride,
     const uint16_t* __restrict__ w, int d, float eps, uint16_t* __restrict__ sum_out,
     uint16_t* __restrict__ out) {
+  constexpr bool kResidual = kRes != Residual::kNone;
   constexpr int kMaxChunks = 4;  // d <= 8 * 256 * 4 = 8192
   __shared__ float red[kNormThreads / kWave];
   const int64_t row = blockIdx.x;
@@ -44,7 +49,20 @@ __global__ __launch_bounds__(kNormThreads) void rms_norm_kernel(
     if (c < n_chunks) {
       u32x4 a = ld16(xr + 8 * c);
       if constexpr (kResidual) {
-        const u32x4 b = ld16(res + row * d + 8 * c);
+        u32x4 b;
+        if constexpr (kRes == Residual::kPartials) {
+          const float* p = part + row * d + 8 * c;
+          f32x4 lo = *reinterpret_cast<const f32x4*>(p), hi = *reinterpret_cast<const f32x4*>(p + 4);
+          for (int sp = 1; sp < n_split; ++sp) {
+            p += stride;
+            lo += *reinterpret_cast<const f32x4*>(p);
+            hi += *reinterpret_cast<const f32x4*>(p + 4);
+          }
+          b = u32x4{pack_bf16x2(lo[0], lo[1]), pack_bf16x2(lo[2], lo[3]),
+                    pack_bf16x2(hi[0], hi[1]), pack_bf16x2(hi[2], hi[3])};
+        } else {
+          b = ld16(res + row * d + 8 * c);
+        }
 #pragma unroll
         for (int j = 0; j < 4; ++j)
           a[j] = pack_bf16x2(bf_lo(a[j]) + bf_lo(b[j]), bf_hi(a[j]) + bf_hi(b[j]));
@@ -196,12 +214,43 @@ extern "C" int fdl_rms_norm(const void* x, const void* residual, const void* wei
   const auto* wp = static_cast<const uint16_t*>(weight);
   auto* sp = static_cast<uint16_t*>(sum_out);
   auto* op = static_cast<uint16_t*>(out);
-  if (residual)
-    hipLaunchKernelGGL(rms_norm_kernel<true>, dim3(static_cast<unsigned>(n_rows)),
-                       dim3(kNormThreads), 0, st, xp, rp, wp, static_cast<int>(d), eps, sp, op);
-  else
-    hipLaunchKernelGGL(rms_norm_kernel<false>, dim3(static_cast<unsigned>(n_rows)),
-                       dim3(kNormThreads), 0, st, xp, rp, wp, static_cast<int>(d), eps, sp, op);
+  hipLaunchKernelGGL((residual ? rms_norm_kernel<Residual::kRows> : rms_norm_kernel<Residual::kNone>),
+                     dim3(static_cast<unsigned>(n_rows)), dim3(kNormThreads), 0, st, xp, rp,
+                     static_cast<const float*>(nullptr), 0, int64_t(0), wp, static_cast<int>(d),
+                     eps, sp, op);
+  FDL_HIP_CHECK(hipGetLastError());
+  return ok();
+}
+
+extern "C" int fdl_rms_norm_partials(const void* x, const float* part, int64_t n_split,
+                                     const void* weight, int64_t n_rows, int64_t d, float eps,
+                                     void* sum_out, void* out, void* stream) {
+  using namespace fdl;
+  FDL_REQUIRE(n_rows >= 0 && n_rows < (int64_t(1) << 31), FDL_ERR_SHAPE,
+              "fdl_rms_norm_partials: n_rows = %lld out of range", (long long)n_rows);
+  FDL_REQUIRE(d >= 8 && d <= 8192 && d % 8 == 0, FDL_ERR_UNSUPPORTED,
+              "fdl_rms_norm_partials: d = %lld (a multiple of 8 up to 8192 is implemented)",
+              (long long)d);
+  FDL_REQUIRE(n_split >= 1 && n_split <= 64, FDL_ERR_UNSUPPORTED,
+              "fdl_rms_norm_partials: n_split = %lld outside [1, 64]", (long long)n_split);
+  FDL_REQUIRE(eps >= 0.f, FDL_ERR_SHAPE, "fdl_rms_norm_partials: eps < 0");
+  if (n_rows == 0) return ok();
+  FDL_REQUIRE_PTR(x);
+  FDL_REQUIRE_PTR(part);
+  FDL_REQUIRE_PTR(weight);
+  FDL_REQUIRE_PTR(sum_out);
+  FDL_REQUIRE_PTR(out);
+  FDL_REQUIRE_ALIGNED(x, 16);
+  FDL_REQUIRE_ALIGNED(part, 16);
+  FDL_REQUIRE_ALIGNED(weight, 16);
+  FDL_REQUIRE_ALIGNED(sum_out, 16);
+  FDL_REQUIRE_ALIGNED(out, 16);
+  hipLaunchKernelGGL(rms_norm_kernel<Residual::kPartials>, dim3(static_cast<unsigned>(n_rows)),
+                     dim3(kNormThreads), 0, static_cast<hipStream_t>(stream),
+                     static_cast<const uint16_t*>(x), static_cast<const uint16_t*>(nullptr), part,
+                     static_cast<int>(n_split), n_rows * d, static_cast<const uint16_t*>(weight),
+                     static_cast<int>(d), eps, static_cast<uint16_t*>(sum_out),
+                     static_cast<uint16_t*>(out));
   FDL_HIP_CHECK(hipGetLastError());
   return ok();
 }

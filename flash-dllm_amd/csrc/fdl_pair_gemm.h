@@ -47,10 +47,11 @@ typedef __attribute__((address_space(3))) void* PgLds;
 typedef __attribute__((address_space(1))) void* PgGlb;
 
 struct PairGemmTiles {
-  const uint16_t* x;  // [n_rows][k]
+  const uint16_t* x;  // [n_rows][ld]
   int64_t n_rows;
-  int k;        // a multiple of 128, at least 256
+  int k;        // reduction length of a workgroup (256-row tiles: a multiple of 128, at least 256)
   int n_mtiles, n_ntiles;
+  int ld;       // row stride of x; the weight rows' is the epilogue's business
 };
 
 // 16 bytes per lane from global memory into LDS at lds + 16 * lane (lds wavefront-uniform),
@@ -177,12 +178,12 @@ __global__ __launch_bounds__((4 + NPROD) * 64, 1) void pair_pc_kernel(PairGemmTi
   const int n_tiles = t.n_mtiles * t.n_ntiles;
   tile_coords(xcd_tile(blockIdx.x, n_tiles), t.n_mtiles, n_tiles, nt, mt);
   const int64_t m0 = int64_t(mt) * BM;
-  const int D = t.k;
+  const int64_t ksplit = int64_t(blockIdx.y) * t.k;  // this part's place in the reduction
   // The wavefront index is uniform; readfirstlane makes the role test a scalar branch, so a
   // wavefront executes only its own role's barriers (both roles execute 3 + nk of them).
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
   const bool producer = wave >= kConsumers;
-  const int nk = D / kPgKT;
+  const int nk = t.k / kPgKT;
 
   // Places of tile rows 0 .. BM - 1 (threads 0 .. BM - 1), found now and staged in LDS for the
   // epilogue once the stage memory is free.
@@ -206,10 +207,10 @@ __global__ __launch_bounds__((4 + NPROD) * 64, 1) void pair_pc_kernel(PairGemmTi
       const int row = 8 * q + (lane >> 3);
       const int c = (lane & 7) ^ ((row >> 1) & 7);
       if (row < BM) {
-        src[i] = t.x + min(m0 + row, t.n_rows - 1) * D + 8 * c;
+        src[i] = t.x + min(m0 + row, t.n_rows - 1) * t.ld + ksplit + 8 * c;
       } else {
         const int wr = row - BM, hlf = wr / BP;
-        src[i] = ep.wrow(BP * nt + (wr - hlf * BP), hlf) + 8 * c;
+        src[i] = ep.wrow(BP * nt + (wr - hlf * BP), hlf) + ksplit + 8 * c;
       }
       dst_off[i] = 1024 * q;
     }
@@ -569,16 +570,19 @@ inline int pg_device_cus() {
 }
 
 // `kernel` of BM-row, BP-pair tiles over n_rows rows and n_pairs pairs (a multiple of BP).
+// n_split > 1 (producer / consumer kernels): part z of the reduction, k / n_split long, runs as
+// grid row z.
 template <class Ep>
 hipError_t pair_launch(void (*kernel)(PairGemmTiles, Ep), int bm, int bp, int threads,
                        const uint16_t* x, int64_t n_rows, int64_t k, int64_t n_pairs, const Ep& ep,
-                       hipStream_t stream) {
+                       hipStream_t stream, int64_t n_split = 1) {
   const int64_t n_mtiles = (n_rows + bm - 1) / bm, n_ntiles = n_pairs / bp;
   if (n_mtiles * n_ntiles >= (int64_t(1) << 31)) return hipErrorInvalidValue;
-  const PairGemmTiles t = {x, n_rows, static_cast<int>(k), static_cast<int>(n_mtiles),
-                           static_cast<int>(n_ntiles)};
-  hipLaunchKernelGGL(kernel, dim3(static_cast<unsigned>(n_mtiles * n_ntiles)), dim3(threads), 0,
-                     stream, t, ep);
+  const PairGemmTiles t = {x, n_rows, static_cast<int>(k / n_split), static_cast<int>(n_mtiles),
+                           static_cast<int>(n_ntiles), static_cast<int>(k)};
+  hipLaunchKernelGGL(kernel,
+                     dim3(static_cast<unsigned>(n_mtiles * n_ntiles), static_cast<unsigned>(n_split)),
+                     dim3(threads), 0, stream, t, ep);
   return hipGetLastError();
 }
 

@@ -126,6 +126,10 @@ SIGNATURES: dict[str, tuple] = {
     "fdl_silu_mul_rows": (ctypes.c_int, [_p, _p, _i64, _i64, _i64, _i64, _p, _p]),
     # x, w_gate, w_up, n_rows, k, width, out_chunks, out, stream
     "fdl_gate_up_silu": (ctypes.c_int, [_p, _p, _p, _i64, _i64, _i64, _i64, _p, _p]),
+    # x, w, n_rows, k, n_out, n_split, transposed, part, stream
+    "fdl_linear_partials": (ctypes.c_int, [_p, _p, _i64, _i64, _i64, _i64, _i32, _p, _p]),
+    # x, part, n_split, weight, n_rows, d, eps, sum_out, out, stream
+    "fdl_rms_norm_partials": (ctypes.c_int, [_p, _p, _i64, _p, _i64, _i64, _f32, _p, _p, _p]),
     "fdl_split_reduce_residual": (ctypes.c_int, [_p, _i64, _i64, _i64, _p, _p]),
     # logits, n_rows, vocab, token, prob, arg, stream
     "fdl_softmax_confidence": (ctypes.c_int, [_p, _i64, _i64, _p, _p, _p, _p]),

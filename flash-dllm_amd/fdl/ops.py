@@ -481,6 +481,45 @@ def gate_up_silu(x: torch.Tensor, w_gate: torch.Tensor, w_up: torch.Tensor,
     return out
 
 
+def linear_partials(x: torch.Tensor, w: torch.Tensor, transposed: bool = False) -> torch.Tensor:
+    """Partial sums [S, rows, n_out] float32 of x w^T over S chunks of the reduction
+    (fdl_linear_partials), for few rows: x [rows, k], w [n_out, k], or with transposed
+    [k, n_out]; k a multiple of 64, n_out of 128. S is the largest of 8, 4, 2, 1 whose workgroups
+    fit the compute units once and whose chunks are multiples of 64 (64 rows, k = n_out = 4096,
+    with the pass that adds the sums: S = 1 / 2 / 4 / 8 take 26 / 19 / 15.6 / 21 us)."""
+    dev = x.device
+    _need(x, "x", BF16, 2)
+    _need(w, "w", BF16, 2, dev)
+    rows, k = x.shape
+    n_out = w.shape[1] if transposed else w.shape[0]
+    if w.shape[0 if transposed else 1] != k:
+        raise _lib.FdlError(_lib.FDL_ERR_SHAPE, f"w has shape {tuple(w.shape)} for {k} columns")
+    tiles = -(-rows // (64 if rows <= 64 else 128)) * (n_out // (128 if transposed else 64))
+    cus = _cus(dev)
+    split = next((s for s in (8, 4, 2) if tiles * s <= cus and k % (64 * s) == 0), 1)
+    part = torch.empty((split, rows, n_out), dtype=torch.float32, device=dev)
+    _lib.call("fdl_linear_partials", x.data_ptr(), w.data_ptr(), rows, k, n_out, split,
+              int(transposed), part.data_ptr(), _stream(x))
+    return part
+
+
+def rms_norm_partials(x: torch.Tensor, weight: torch.Tensor, eps: float, part: torch.Tensor):
+    """(s, RMSLayerNorm of s times weight) with s = bf16(x + bf16(sum_z part[z]))
+    (fdl_rms_norm_partials): rms_norm whose residual comes as partial sums."""
+    dev = x.device
+    _need(x, "x", BF16, 2)
+    n_rows, d = x.shape
+    _need(weight, "weight", BF16, 1, dev)
+    _need(part, "part", torch.float32, 3, dev)
+    if weight.shape[0] != d or tuple(part.shape[1:]) != (n_rows, d):
+        raise _lib.FdlError(_lib.FDL_ERR_SHAPE, "part must be [S, rows, d] and weight [d]")
+    sum_out, out = torch.empty_like(x), torch.empty_like(x)
+    _lib.call("fdl_rms_norm_partials", x.data_ptr(), part.data_ptr(), part.shape[0],
+              weight.data_ptr(), n_rows, d, float(eps), sum_out.data_ptr(), out.data_ptr(),
+              _stream(x))
+    return sum_out, out
+
+
 def split_reduce_residual(part: torch.Tensor, residual: torch.Tensor) -> torch.Tensor:
     """residual = bf16(residual + sum_s part[s]) in place (fdl_split_reduce_residual):
     part fp32 [S, rows, cols], residual bf16 [rows, cols]."""

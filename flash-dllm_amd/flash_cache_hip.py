@@ -157,6 +157,48 @@ def _adjacent_gate_up(block) -> torch.Tensor | None:
     return torch.as_strided(wg, (2 * h, d), (d, 1))
 
 
+def _plain_linear(m) -> bool:
+    """A torch.nn.Linear with a plain contiguous bf16 GPU weight, without bias or hooks: its
+    product may run without calling the module."""
+    w = getattr(m, "weight", None)
+    return (type(m) is torch.nn.Linear and m.bias is None and not m._forward_hooks
+            and not m._forward_pre_hooks and type(w) in (torch.nn.Parameter, torch.Tensor)
+            and w.dtype == torch.bfloat16 and w.is_cuda and w.is_contiguous()
+            and w.data_ptr() % 16 == 0)
+
+
+# Few rows leave a product without enough tiles for the device; cut over the reduction, with the
+# partial sums added by the next pass (norm or residual), its weights stream through every
+# compute unit. attn_out with the norm behind it, cold weights (us), library product / parts:
+# d_model 4096: 16 rows 19.5 / 14.4, 64 rows 19.8 / 15.6, 128 rows 28.7 / 18.8, 256 rows 27.0 /
+# 23.2 (512 rows: as many tiles as the library's); d_model 2048: 64 rows 12.0 / 10.0, 128 rows
+# 11.7 / 11.8, 256 rows 13.0 / 14.6. ff_out (k 12288) with the residual pass: 16 rows 26.5 / 26.2,
+# 64 rows 30.2 / 28.4, 128 rows 39.0 / 36.6, 256 rows 51 / 55; k 6144, d_model 2048: 16 rows 11.8 /
+# 14.0, 128 rows 16.3 / 21.3 (the library's four parts suffice). Each product also saves about
+# 10 us of library set-up on the host.
+PARTS_MAX_ROWS = 128
+PARTS_WIDE_WEIGHT = 1 << 24          # elements from which attn_out takes twice the rows
+PARTS_FF_OUT_WEIGHT = 1 << 25        # elements from which ff_out runs in parts
+
+
+def _attn_out_in_parts(m, x: torch.Tensor, att: torch.Tensor) -> bool:
+    if not (_plain_linear(m) and att.dim() == 2 and att.dtype == torch.bfloat16 and att.is_cuda
+            and att.is_contiguous() and att.data_ptr() % 16 == 0):
+        return False
+    n_out, k = m.weight.shape
+    rows = att.shape[0]
+    return (0 < rows <= PARTS_MAX_ROWS * (2 if n_out * k >= PARTS_WIDE_WEIGHT else 1)
+            and k % 64 == 0 and n_out % 128 == 0 and tuple(x.shape) == (rows, n_out)
+            and att.shape[1] == k)
+
+
+def _ff_out_in_parts(w: torch.Tensor, rows: int) -> bool:
+    """For an ff_out that the split-K product takes (weight stored transposed)."""
+    n_out, k = w.shape
+    return (rows <= PARTS_MAX_ROWS and n_out * k >= PARTS_FF_OUT_WEIGHT and k % 64 == 0
+            and n_out % 128 == 0 and w.data_ptr() % 16 == 0)
+
+
 def _fused_gate_up(x: torch.Tensor, w_gu: torch.Tensor) -> bool:
     """Whether the gate and up products and the SiLU gate run as one kernel
     (ops.gate_up_silu): the shapes it takes, at row counts where it is the faster way."""
@@ -208,11 +250,17 @@ def _ff_out_residual(block, x: torch.Tensor, og_x: torch.Tensor) -> torch.Tensor
 
 def block_mlp_tail(self, x: torch.Tensor, att: torch.Tensor) -> torch.Tensor:
     """attn_out + residual + SiLU-gated MLP + residual (flash_cache_triton.py:618-638)."""
-    att = self.attn_out(att)
     ck = self._activation_checkpoint_fn
     p = _rms_params(self.ff_norm) if ck is None else None
-    if (p is not None and _identity_dropout(self.dropout) and x.dtype == torch.bfloat16
-            and att.dtype == torch.bfloat16):
+    fuse_norm = p is not None and _identity_dropout(self.dropout) and x.dtype == torch.bfloat16
+    parts = fuse_norm and _attn_out_in_parts(self.attn_out, x, att)
+    if not parts:
+        att = self.attn_out(att)
+    if parts:
+        # the product's partial sums, added by the pass below
+        og_x, x = ops.rms_norm_partials(x.contiguous(), p[0], p[1],
+                                        ops.linear_partials(att, self.attn_out.weight))
+    elif fuse_norm and att.dtype == torch.bfloat16:
         # x + dropout(att) and ff_norm in one pass
         og_x, x = ops.rms_norm(x.contiguous(), p[0], p[1], residual=att.contiguous())
     else:
@@ -227,13 +275,18 @@ def block_mlp_tail(self, x: torch.Tensor, att: torch.Tensor) -> torch.Tensor:
         h = self.ff_proj.weight.shape[0]
         ws = _split_k_ff_out(self, x.shape[0])
         split = ws is not None and og_x.is_contiguous() and og_x.dtype == torch.bfloat16
-        # SiLU(gate) * up written as the K-chunks [S, rows, K / S] of a split-K ff_out
-        chunks = ws.shape[0] if split else 1
+        in_parts = split and _ff_out_in_parts(self.ff_out.weight, x.shape[0])
+        # SiLU(gate) * up written as the K-chunks [S, rows, K / S] of a batched split-K ff_out
+        chunks = ws.shape[0] if split and not in_parts else 1
         if _fused_gate_up(x, w_gu):
             x = ops.gate_up_silu(x, w_gu[:h], w_gu[h:], out_chunks=chunks)
         else:
             gu = F.linear(x, w_gu)
             x = ops.silu_mul(gu[:, :h], gu[:, h:], out_chunks=chunks)
+        if in_parts:
+            return ops.split_reduce_residual(
+                ops.linear_partials(x, self.ff_out.weight.t(), transposed=True),
+                og_x).unsqueeze(0)
         if split:
             # the batched product's right operands are contiguous chunks of W^T; partials +
             # residual in one pass

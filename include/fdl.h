@@ -301,6 +301,24 @@ int fdl_gate_up_silu(const void* x, const void* w_gate, const void* w_up, int64_
                      int64_t k, int64_t width, int64_t out_chunks, void* out, void* stream);
 
 /*
+ * A product cut over its reduction, for few rows (attn_out and ff_out, flash_cache_triton.py:618,
+ * :634): part[z][r][n] = sum over k in chunk z of x[r][k] * w[n][k], fp32 [n_split][n_rows][n_out],
+ * to be added by fdl_rms_norm_partials or fdl_split_reduce_residual. x [n_rows][k] bf16; w
+ * [n_out][k], or with `transposed` [k][n_out]. k: n_split chunks of a multiple of 64; n_out: a
+ * multiple of 128; all pointers 16-byte aligned.
+ */
+int fdl_linear_partials(const void* x, const void* w, int64_t n_rows, int64_t k, int64_t n_out,
+                        int64_t n_split, int32_t transposed, float* part, void* stream);
+
+/*
+ * fdl_rms_norm with the residual as n_split fp32 partial sums [n_split][n_rows][d], added in
+ * ascending order and rounded to bf16 before the residual add.
+ */
+int fdl_rms_norm_partials(const void* x, const float* part, int64_t n_split, const void* weight,
+                          int64_t n_rows, int64_t d, float eps, void* sum_out, void* out,
+                          void* stream);
+
+/*
  * fdl_split_reduce_residual: the end of a split-K ff_out product with its residual
  * (flash_cache_triton.py:634-636, `x = og_x + ff_out(x)`):
  *   residual_out[i] = bf16(float(residual_out[i]) + (part[0][i] + part[1][i] + ...)),

@@ -86,6 +86,14 @@ def test_launchers_reject_bad_scalars_without_gpu():
         _expect(lib.FDL_ERR_UNSUPPORTED, "fdl_gate_up_silu", None, None, None, 4, k, width, chunks,
                 None, None)
     _expect(lib.FDL_ERR_NULL, "fdl_gate_up_silu", None, None, None, 4, 256, 96, 1, None, None)
+    for k, n_out, split in ((96, 128, 1), (128, 128, 4), (64, 64, 1), (64, 128, 0)):
+        _expect(lib.FDL_ERR_UNSUPPORTED, "fdl_linear_partials", None, None, 4, k, n_out, split, 0,
+                None, None)
+    _expect(lib.FDL_ERR_NULL, "fdl_linear_partials", None, None, 4, 64, 128, 1, 0, None, None)
+    _expect(lib.FDL_ERR_UNSUPPORTED, "fdl_rms_norm_partials", None, None, 0, None, 4, 64, 1e-5, None,
+            None, None)
+    _expect(lib.FDL_ERR_NULL, "fdl_rms_norm_partials", None, None, 2, None, 4, 64, 1e-5, None, None,
+            None)
     lib.call("fdl_gate_up_silu", None, None, None, 0, 256, 96, 1, None, None)  # zero rows: no-op
     _expect(lib.FDL_ERR_UNSUPPORTED, "fdl_split_reduce_residual", None, 0, 4, 16, None, None)
     _expect(lib.FDL_ERR_UNSUPPORTED, "fdl_split_reduce_residual", None, 4, 4, 12, None, None)

@@ -188,3 +188,42 @@ def test_gate_up_silu_matches_unfused(rows, k, width, chunks):
     tol = ref.float().abs() * (2.0**-8 * (2 + g.float().abs()) + 2.0**-7) + 1e-3
     assert bool(((got.float() - ref.float()).abs() <= tol).all())
     assert (got != ref).float().mean() < 0.02
+
+
+@pytest.mark.parametrize("transposed", [False, True])
+@pytest.mark.parametrize("rows,k,n_out", [(1, 64, 128), (64, 512, 256), (65, 192, 128), (128, 4096, 384),
+                                          (129, 576, 256), (40, 12288, 4096), (200, 1024, 4096)])
+def test_linear_partials_and_the_passes_that_add_them(rows, k, n_out, transposed):
+    """Partial sums against float64 (fp32 sums of k terms: 2^-24 sqrt(k) of the terms' 2-norm,
+    with a factor 8), and the norm over them bit for bit the norm over their bf16 sum."""
+    gen = torch.Generator().manual_seed(rows + k)
+    x = torch.randn(rows, k, generator=gen).to(torch.bfloat16).to(DEV)
+    w = (torch.randn(n_out, k, generator=gen) * 0.05).to(torch.bfloat16).to(DEV)
+    part = ops.linear_partials(x, w.t().contiguous() if transposed else w, transposed=transposed)
+    assert part.dtype == torch.float32 and tuple(part.shape[1:]) == (rows, n_out)
+    ref = x.double().cpu() @ w.double().cpu().t()
+    scale = (x.double().cpu() ** 2) @ (w.double().cpu() ** 2).t()
+    err = (part.double().cpu().sum(0) - ref).abs()
+    assert bool((err <= 8 * 2.0**-24 * k**0.5 * scale.sqrt() + 1e-12).all())
+    h = torch.randn(rows, n_out, generator=gen).to(torch.bfloat16).to(DEV)
+    nw = torch.randn(n_out, generator=gen).to(torch.bfloat16).to(DEV)
+    total = part[0].clone()
+    for p in part[1:]:
+        total += p
+    ref_s, ref_y = ops.rms_norm(h, nw, 1e-5, residual=total.to(torch.bfloat16))
+    got_s, got_y = ops.rms_norm_partials(h, nw, 1e-5, part)
+    assert torch.equal(got_s, ref_s) and torch.equal(got_y, ref_y)
+
+
+def test_attn_out_with_hooks_is_called_as_a_module():
+    """A module with a hook, a bias or another class is called; a plain one runs in parts."""
+    import flash_cache_hip as fch
+    m = torch.nn.Linear(256, 256, bias=False, device=DEV, dtype=torch.bfloat16)
+    x = torch.randn(8, 256, device=DEV).to(torch.bfloat16)
+    assert fch._attn_out_in_parts(m, x, x)
+    hook = m.register_forward_hook(lambda *a: None)
+    assert not fch._attn_out_in_parts(m, x, x)
+    hook.remove()
+    assert not fch._attn_out_in_parts(torch.nn.Linear(256, 256, device=DEV, dtype=torch.bfloat16), x, x)
+    assert not fch._attn_out_in_parts(m, x, x.t().contiguous().t())
+    assert not fch._attn_out_in_parts(m, x[:, :128], x)
