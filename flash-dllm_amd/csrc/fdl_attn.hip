@@ -720,6 +720,9 @@ __global__ __launch_bounds__(64 * (NC + kProducers), 1) void attn_kernel(AttnArg
     vS = a.vmeta[2 * vb_idx + 1];
   }
   const bool wave_imp = 16 * RB * wr < n_imp;
+  // a consumer without rows only keeps the barriers (tiles of up to 64 rows in a launch of
+  // 128-row tiles); softmax importance reads every consumer's probabilities
+  const bool no_rows = !kVerify && NC == 8 && !imp_soft && 16 * RB * wr >= n_rows;
   const int imp_waves = (n_imp + 16 * RB - 1) / (16 * RB);
   float lse_r[RB][4];
 
@@ -846,7 +849,7 @@ __global__ __launch_bounds__(64 * (NC + kProducers), 1) void attn_kernel(AttnArg
           for (int ii = 0; ii < 4; ++ii)
             kbias[kb][ii] = 16 * kb + 4 * g + ii < n_left ? 0.f : -INFINITY;
         const int blk = block_of(s);
-        attend_block<RB>(
+        if (!no_rows) attend_block<RB>(
             st, qf, kt, vt, a.scale_log2, [&](int, int kb, int ii) { return kbias[kb][ii]; },
             [&](int rb, const f32x4 (&p)[4], float m_use) {
               const int r = 16 * (wr * RB + rb) + l16;

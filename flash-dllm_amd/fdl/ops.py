@@ -181,6 +181,24 @@ def _split_parts(plan: AttnPlan, first: int, count: int, tile_rows: int, n_heads
     return parts if parts >= 2 else 0
 
 
+def _launch_ranges(plan: AttnPlan, n_heads: int, cus: int, imp_mode: int, key_split: bool):
+    """The launches of a plan, as _class_ranges: mid and short tiles in one launch of 128-row
+    tiles where neither class is split over its keys. Both stream K and V, and a launch for each
+    leaves a part of the device idle in its last round of workgroups twice (96 mid and 160 short
+    workgroups of 512-1024 keys: 25 + 24 us apart, 27 us together; 224 and 608 workgroups of
+    512-1536 keys: 44 + 88 us, 108 us). A short tile's rows are computed alike in both. Softmax-
+    colsum importance keeps its probabilities on chip in 64-row launches only, so it keeps the
+    classes apart."""
+    ranges = _class_ranges(plan)
+    (_, _, _), (m0, n_mid, mid_rows), (s0, n_short, short_rows) = ranges
+    if n_mid == 0 or n_short == 0 or imp_mode == _lib.IMP_SOFTMAX_COLSUM:
+        return ranges
+    if key_split and (_split_parts(plan, m0, n_mid, mid_rows, n_heads, cus)
+                      or _split_parts(plan, s0, n_short, short_rows, n_heads, cus)):
+        return ranges
+    return ranges[0], (m0, n_mid + n_short, mid_rows)
+
+
 def attention_split_floats(plan: AttnPlan, n_heads: int, cus: int) -> int:
     """fp32 workspace for fdl_block_attention's key split (no or raw importance): the largest
     class need of _split_parts workgroups per tile, each writing ATTN_PART_FLOATS floats per
@@ -237,7 +255,7 @@ def block_attention(q: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tenso
         _need(workspace, "workspace", torch.float32, 1, dev)
     # long tiles (the first n_long work items), mid tiles (the next n_mid), short tiles
     cus = _cus(dev)
-    for first, count, tile_rows in _class_ranges(plan):
+    for first, count, tile_rows in _launch_ranges(plan, n_heads, cus, imp_mode, key_split):
         if count == 0:
             continue
         ws_n = 0 if workspace is None else workspace.numel()

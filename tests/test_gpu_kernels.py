@@ -1119,3 +1119,43 @@ def test_verify_attention_random_blocks(seed):
     got = _np(out)
     _close(got[:acc_q], ref[:acc_q], what=f"verify attention, seed {seed}")
     assert np.all(got[acc_q:] == POISON)
+
+
+@pytest.mark.parametrize("imp_mode", [lib.IMP_NONE, lib.IMP_RAW_LOGIT])
+def test_mid_and_short_tiles_in_one_launch_equal_two(imp_mode, monkeypatch):
+    """Mid (65-128 row) and short tiles of one plan run in one launch of 128-row tiles; the
+    result is bit for bit that of a launch per class, over row counts at the tiles' edges and
+    key counts past the staged slot map."""
+    rng = np.random.default_rng(21)
+    H, P, n_q = 32, 32, [1, 16, 17, 48, 63, 64, 65, 80, 127, 128, 33, 100]
+    k_ends = [97, 640, 64, 2100, 33, 700, 500, 2080, 129, 900, 1, 300]
+    seqs, q0 = [], 0
+    for b, (n, k) in enumerate(zip(n_q, k_ends)):
+        seqs.append(SeqRows(batch=b, k_end=k, rows=np.arange(q0, q0 + n),
+                            n_imp=min(n, 32) if imp_mode else 0))
+        q0 += n
+    pages = [-(-k // P) for k in k_ends]
+    table, nxt = np.zeros((len(seqs), max(pages)), np.int32), 0
+    perm = rng.permutation(sum(pages))
+    for b, n in enumerate(pages):
+        table[b, :n] = perm[nxt:nxt + n]
+        nxt += n
+    q, kc, vc = (t.to(DEV) for t in _attn_inputs(22, q0, sum(pages) * P, H))
+    plan = make_plan(seqs, table, 5, device=DEV)
+    cus = torch.cuda.get_device_properties(DEV).multi_processor_count
+    assert plan.n_long == 0 and plan.n_mid == 5 and plan.n_work == 12
+    assert len(ops._launch_ranges(plan, H, cus, imp_mode, False)) == 2
+    assert len(ops._launch_ranges(plan, H, cus, lib.IMP_SOFTMAX_COLSUM, False)) == 3
+
+    def run():
+        out = torch.full((q0, H * 128), POISON, dtype=torch.bfloat16, device=DEV)
+        imp = torch.zeros((H, sum(pages) * P), dtype=torch.float32, device=DEV)
+        ops.block_attention(q, kc, vc, plan, out, H, orc.softmax_scale(128), imp_mode,
+                            imp if imp_mode else None, key_split=False)
+        return out, imp
+
+    one = run()
+    monkeypatch.setattr(ops, "_launch_ranges", lambda p, *_: ops._class_ranges(p))
+    two = run()
+    assert torch.equal(one[0], two[0]) and torch.equal(one[1], two[1])
+    assert not bool((one[0] == POISON).all(1).any())
