@@ -25,6 +25,8 @@ import torch
 import torch.nn as nn
 import torch.nn.functional as F
 
+from . import ops
+
 
 @dataclass
 class LLaDAConfig:
@@ -142,6 +144,21 @@ class LLaDALlamaBlock(nn.Module):
                               positions=positions, lengths=lengths), None
 
 
+def _final_norm(norm: nn.Module, x: torch.Tensor) -> torch.Tensor:
+    """norm(x); a plain RMSLayerNorm of bf16 GPU rows in one pass (fdl_rms_norm) instead of
+    eight: 35 -> 5 us at 256 rows of 4096. Under autograd, and with hooks, the module is called."""
+    d = x.shape[-1]
+    w = getattr(norm, "weight", None)
+    if not (type(norm) is RMSLayerNorm and x.is_cuda and x.dtype == w.dtype == torch.bfloat16
+            and w.device == x.device and w.dim() == 1 and w.is_contiguous()
+            and (x.data_ptr() | w.data_ptr()) % 16 == 0 and d % 8 == 0 and 8 <= d <= 8192
+            and x.numel() > 0
+            and not norm._forward_hooks and not norm._forward_pre_hooks
+            and not (torch.is_grad_enabled() and (x.requires_grad or w.requires_grad))):
+        return norm(x)
+    return ops.rms_norm(x.reshape(-1, d).contiguous(), w, norm.eps).view(x.shape)
+
+
 class LLaDAModel(nn.Module):
     def __init__(self, cfg: LLaDAConfig, attention_fn: Callable, device=None, dtype=None):
         super().__init__()
@@ -163,7 +180,7 @@ class LLaDAModel(nn.Module):
         if logit_rows is not None:
             # only the rows the scheduler reads (same values, fewer vocab GEMM rows)
             x = x[:, logit_rows]
-        x = self.transformer.ln_f(x)
+        x = _final_norm(self.transformer.ln_f, x)
         return self.transformer.ff_out(x)
 
 

@@ -227,3 +227,18 @@ def test_attn_out_with_hooks_is_called_as_a_module():
     assert not fch._attn_out_in_parts(torch.nn.Linear(256, 256, device=DEV, dtype=torch.bfloat16), x, x)
     assert not fch._attn_out_in_parts(m, x, x.t().contiguous().t())
     assert not fch._attn_out_in_parts(m, x[:, :128], x)
+
+
+@pytest.mark.parametrize("rows", [1, 37])
+def test_final_norm_matches_module(rows):
+    """The model's final norm in one kernel against the module (the bounds of the norm kernel's
+    own test), and the module itself under autograd."""
+    from fdl.model import _final_norm
+    norm = RMSLayerNorm(512, 1e-5, DEV, torch.bfloat16)
+    x = torch.randn(1, rows, 512, device=DEV).to(torch.bfloat16)
+    with torch.no_grad():
+        norm.weight.normal_()
+        got = _final_norm(norm, x)
+        assert got.shape == x.shape
+        _check(got, norm(x), f"final norm {rows}")
+    assert _final_norm(norm, x).requires_grad
