@@ -189,7 +189,7 @@ def load() -> ctypes.CDLL:
 
 def call(name: str, *args) -> None:
     """Calls entry point `name`; raises FdlError with the library's message on failure."""
-    lib = load()
+    lib = _lib or load()
     status = getattr(lib, name)(*args)
     if status != FDL_OK:
         msg = lib.fdl_last_error().decode(errors="replace")

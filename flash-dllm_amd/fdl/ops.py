@@ -31,6 +31,12 @@ def _stream(t: torch.Tensor) -> int:
 
 def _need(t: torch.Tensor, name: str, dtype: torch.dtype, ndim: int | None = None,
           device: torch.device | None = None) -> None:
+    # the usual case first: a launch checks up to ten tensors (a 40-row projection 11.3 -> 9.4 us of
+    # host time)
+    if (isinstance(t, torch.Tensor) and t.is_cuda and t.dtype is dtype
+            and (ndim is None or t.ndim == ndim) and (device is None or t.device == device)
+            and t.is_contiguous()):
+        return
     if not isinstance(t, torch.Tensor):
         raise TypeError(f"{name} must be a tensor")
     if t.device.type != "cuda":
@@ -182,21 +188,21 @@ def _split_parts(plan: AttnPlan, first: int, count: int, tile_rows: int, n_heads
 
 
 def _launch_ranges(plan: AttnPlan, n_heads: int, cus: int, imp_mode: int, key_split: bool):
-    """The launches of a plan, as _class_ranges: mid and short tiles in one launch of 128-row
-    tiles where neither class is split over its keys. Both stream K and V, and a launch for each
-    leaves a part of the device idle in its last round of workgroups twice (96 mid and 160 short
-    workgroups of 512-1024 keys: 25 + 24 us apart, 27 us together; 224 and 608 workgroups of
-    512-1536 keys: 44 + 88 us, 108 us). A short tile's rows are computed alike in both. Softmax-
-    colsum importance keeps its probabilities on chip in 64-row launches only, so it keeps the
-    classes apart."""
-    ranges = _class_ranges(plan)
-    (_, _, _), (m0, n_mid, mid_rows), (s0, n_short, short_rows) = ranges
-    if n_mid == 0 or n_short == 0 or imp_mode == _lib.IMP_SOFTMAX_COLSUM:
-        return ranges
-    if key_split and (_split_parts(plan, m0, n_mid, mid_rows, n_heads, cus)
-                      or _split_parts(plan, s0, n_short, short_rows, n_heads, cus)):
-        return ranges
-    return ranges[0], (m0, n_mid + n_short, mid_rows)
+    """The launches of a plan, (first, count, tile_rows, key-split parts): its classes, mid and
+    short tiles in one launch of 128-row tiles where neither class is split over its keys. Both
+    stream K and V, and a launch for each leaves a part of the device idle in its last round of
+    workgroups twice (96 mid and 160 short workgroups of 512-1024 keys: 25 + 24 us apart, 27 us
+    together; 224 and 608 workgroups of 512-1536 keys: 44 + 88 us, 108 us). A short tile's rows are
+    computed alike in both. Softmax-colsum importance keeps its probabilities on chip in 64-row
+    launches only, so it keeps the classes apart."""
+    split = key_split and imp_mode != _lib.IMP_SOFTMAX_COLSUM
+    ranges = [(first, count, rows, _split_parts(plan, first, count, rows, n_heads, cus) if split else 0)
+              for first, count, rows in _class_ranges(plan)]
+    (_, _, _, _), (m0, n_mid, mid_rows, mid_parts), (_, n_short, _, short_parts) = ranges
+    if (n_mid and n_short and not mid_parts and not short_parts
+            and imp_mode != _lib.IMP_SOFTMAX_COLSUM):
+        return ranges[0], (m0, n_mid + n_short, mid_rows, 0)
+    return ranges
 
 
 def attention_split_floats(plan: AttnPlan, n_heads: int, cus: int) -> int:
@@ -247,24 +253,22 @@ def block_attention(q: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tenso
     if imp_mode == _lib.IMP_SOFTMAX_COLSUM and workspace is None:
         workspace = torch.empty(max(attention_workspace_floats(plan, n_heads), 4),
                                 dtype=torch.float32, device=dev)
-    elif imp_mode != _lib.IMP_SOFTMAX_COLSUM and workspace is None and key_split:
-        n = attention_split_floats(plan, n_heads, _cus(dev))
+    # long tiles (the first n_long work items), mid tiles (the next n_mid), short tiles
+    ranges = _launch_ranges(plan, n_heads, _cus(dev), imp_mode, key_split)
+    part_floats = n_row_idx * n_heads * _lib.ATTN_PART_FLOATS  # one part's room
+    if workspace is None:
+        n = max(parts for _, _, _, parts in ranges) * part_floats
         if n:
             workspace = torch.empty(n, dtype=torch.float32, device=dev)
     if workspace is not None:
         _need(workspace, "workspace", torch.float32, 1, dev)
-    # long tiles (the first n_long work items), mid tiles (the next n_mid), short tiles
-    cus = _cus(dev)
-    for first, count, tile_rows in _launch_ranges(plan, n_heads, cus, imp_mode, key_split):
+    for first, count, tile_rows, parts in ranges:
         if count == 0:
             continue
         ws_n = 0 if workspace is None else workspace.numel()
-        if imp_mode != _lib.IMP_SOFTMAX_COLSUM and key_split:
-            # the room of this class's own parts (the launcher splits as far as the room allows)
-            ws_n = min(ws_n, _split_parts(plan, first, count, tile_rows, n_heads, cus) *
-                       n_row_idx * n_heads * _lib.ATTN_PART_FLOATS)
-        elif imp_mode != _lib.IMP_SOFTMAX_COLSUM:
-            ws_n = 0
+        if imp_mode != _lib.IMP_SOFTMAX_COLSUM:
+            # the room of this launch's own parts (the launcher splits as far as the room allows)
+            ws_n = min(ws_n, parts * part_floats)
         _lib.call("fdl_block_attention", q.data_ptr(), k_cache.data_ptr(), v_cache.data_ptr(),
                   q.shape[0], k_cache.shape[0], d_model, n_heads, d_model // n_heads,
                   plan.page_table_d.data_ptr(), plan.page_table.shape[0], plan.page_table.shape[1],
