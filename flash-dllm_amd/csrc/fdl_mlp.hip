@@ -252,16 +252,16 @@ struct GuCall {
   hipStream_t stream;
 };
 
-template <int BM, int BP, int STAGES, int WM>
+template <int BM, int BP, int NPROD, int STAGES, int WM>
 hipError_t gu_pc(const GuCall& c, int64_t n) {
-  return pair_launch(pair_pc_kernel<SiluEp, BM, BP, 4, STAGES, WM>, BM, BP,
-                     PcShape<BM, BP, 4, STAGES, WM>::kThreads, c.x, n, c.k, c.width, c.ep,
+  return pair_launch(pair_pc_kernel<SiluEp, BM, BP, NPROD, STAGES, WM>, BM, BP,
+                     PcShape<BM, BP, NPROD, STAGES, WM>::kThreads, c.x, n, c.k, c.width, c.ep,
                      c.stream);
 }
 
-// Up to 128 rows the weights stream: 32 pairs a workgroup while that is one round of
-// workgroups, else 48 (width 12288: 256 workgroups; 32 pairs make one and a half rounds, 51.6
-// us at 64 rows against 46.4). Then 128-row tiles while they fit one round (256 rows of width
+// Up to 128 rows the weights stream: 24 pairs a workgroup while that is one round of
+// workgroups (width 6144 at 64 rows: 13.4 us, 32 pairs 14.5), else 48 (width 12288: 256
+// workgroups; 32 pairs make one and a half rounds, 51.6 us at 64 rows against 46.4). Then 128-row tiles while they fit one round (256 rows of width
 // 12288: 61 us, 256-row tiles 85), then 256-row tiles. Against a library product over both
 // weights and a separate SiLU pass, k 4096, width 12288, cold weights (us): 64 rows 50.3 ->
 // 37.1, 128 rows 53.5 -> 45.3, 256 rows 67 -> 61, 384 rows 87 -> 93, 512 rows 98 -> 95, 640 rows
@@ -270,11 +270,11 @@ hipError_t gu_pc(const GuCall& c, int64_t n) {
 hipError_t gu_launch(const GuCall& c, int64_t n) {
   const int64_t cus = pg_device_cus();
   if (n <= 128) {
-    const bool narrow = c.width / 32 <= cus;
-    if (n <= 64) return narrow ? gu_pc<64, 32, 8, 2>(c, n) : gu_pc<64, 48, 8, 4>(c, n);
-    return narrow ? gu_pc<128, 32, 6, 2>(c, n) : gu_pc<128, 48, 5, 4>(c, n);
+    const bool narrow = c.width / 24 <= cus;
+    if (n <= 64) return narrow ? gu_pc<64, 24, 2, 8, 4>(c, n) : gu_pc<64, 48, 4, 8, 4>(c, n);
+    return narrow ? gu_pc<128, 24, 2, 6, 4>(c, n) : gu_pc<128, 48, 4, 5, 4>(c, n);
   }
-  if ((n + 127) / 128 * (c.width / 96) <= cus) return gu_pc<128, 96, 4, 2>(c, n);
+  if ((n + 127) / 128 * (c.width / 96) <= cus) return gu_pc<128, 96, 4, 4, 2>(c, n);
   return pair_launch(pair_gemm_kernel<SiluEp>, kPgBM, kPgBP, kPgThreads, c.x, n, c.k, c.width,
                      c.ep, c.stream);
 }

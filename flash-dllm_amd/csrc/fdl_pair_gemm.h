@@ -144,12 +144,12 @@ __device__ __forceinline__ void pg_barrier() { asm volatile("s_barrier" ::: "mem
 
 // ---------------------------------------------------------------------------------------
 // Shape of one pair_pc_kernel instance. Consumer (wm, wn) of the WM x (4 / WM) consumers owns
-// rows BM/WM * wm .. + BM/WM and pairs kWP * wn .. + kWP (low and high columns).
+// rows BM/WM * wm .. + BM/WM and columns kCols * wn .. + kCols, counted over [BP low | BP high].
 template <int BM, int BP, int NPROD, int STAGES, int WM>
 struct PcShape {
   static constexpr int kConsumers = 4, kWN = kConsumers / WM;
   static constexpr int kThreads = (kConsumers + NPROD) * 64;
-  static constexpr int kWP = BP / kWN, kPB = kWP / 16, kRB = BM / (16 * WM);
+  static constexpr int kCols = 2 * BP / kWN, kCB = kCols / 16, kRB = BM / (16 * WM);
   static constexpr int kABytes = BM * 128;                 // X tile of one step
   static constexpr int kStageBytes = kABytes + 2 * BP * 128;  // + W tile (low, high columns)
   static constexpr int kLoads = kStageBytes / 1024 / NPROD;   // 1 KB loads per producer/step
@@ -157,7 +157,8 @@ struct PcShape {
   // of [BP low | BP high] columns (row stride padded by 4 floats), then the rows' places.
   static constexpr int kEpStride = 2 * BP + 4;
   static constexpr int kEpMetaOff = BM * kEpStride * 4;
-  static_assert(kPB >= 1 && kRB >= 1 && kPB * 16 * kWN == BP && kRB * 16 * WM == BM, "tile shape");
+  static_assert(kCB >= 1 && kRB >= 1 && kCB * 16 * kWN == 2 * BP && kRB * 16 * WM == BM && BP % 8 == 0,
+                "tile shape");
   static_assert(kLoads * NPROD * 1024 == kStageBytes, "producer split");
   static_assert((STAGES - 1) * kLoads < 64, "vmcnt range");
   static_assert(STAGES * kStageBytes <= 160 * 1024, "LDS");
@@ -168,7 +169,7 @@ struct PcShape {
 template <class Ep, int BM, int BP, int NPROD, int STAGES, int WM>
 __global__ __launch_bounds__((4 + NPROD) * 64, 1) void pair_pc_kernel(PairGemmTiles t, Ep ep) {
   using Sh = PcShape<BM, BP, NPROD, STAGES, WM>;
-  constexpr int kWP = Sh::kWP, kPB = Sh::kPB, kRB = Sh::kRB, kLoads = Sh::kLoads;
+  constexpr int kCols = Sh::kCols, kCB = Sh::kCB, kRB = Sh::kRB, kLoads = Sh::kLoads;
   constexpr int kStageBytes = Sh::kStageBytes, kEpStride = Sh::kEpStride;
   constexpr int kThreads = Sh::kThreads, kConsumers = Sh::kConsumers;
   __shared__ __align__(1024) uint8_t smem[STAGES * kStageBytes];
@@ -261,7 +262,7 @@ __global__ __launch_bounds__((4 + NPROD) * 64, 1) void pair_pc_kernel(PairGemmTi
     const int sw = (l16 >> 1) & 7;
     struct Frag {
       u32x4 a[kRB];
-      u32x4 b[2][kPB];
+      u32x4 b[kCB];
     };
     // MFMA operands of half-step ss of the step in `stage`: lane (l16, g4) takes logical
     // chunk 4 ss + g4 of its row.
@@ -271,29 +272,23 @@ __global__ __launch_bounds__((4 + NPROD) * 64, 1) void pair_pc_kernel(PairGemmTi
 #pragma unroll
       for (int rb = 0; rb < kRB; ++rb) f.a[rb] = st[((BM / WM) * wm + 16 * rb + l16) * 8 + c];
 #pragma unroll
-      for (int h = 0; h < 2; ++h)
-#pragma unroll
-        for (int pb = 0; pb < kPB; ++pb)
-          f.b[h][pb] = st[Sh::kABytes / 16 + (BP * h + kWP * wn + 16 * pb + l16) * 8 + c];
+      for (int cb = 0; cb < kCB; ++cb)
+        f.b[cb] = st[Sh::kABytes / 16 + (kCols * wn + 16 * cb + l16) * 8 + c];
     };
-    f32x4 acc[kRB][2][kPB];
+    f32x4 acc[kRB][kCB];
 #pragma unroll
     for (int rb = 0; rb < kRB; ++rb)
 #pragma unroll
-      for (int h = 0; h < 2; ++h)
-#pragma unroll
-        for (int pb = 0; pb < kPB; ++pb) acc[rb][h][pb] = f32x4{0.f, 0.f, 0.f, 0.f};
+      for (int cb = 0; cb < kCB; ++cb) acc[rb][cb] = f32x4{0.f, 0.f, 0.f, 0.f};
     auto mma = [&](const Frag& f) {
 #pragma unroll
       for (int rb = 0; rb < kRB; ++rb)
 #pragma unroll
-        for (int h = 0; h < 2; ++h)
-#pragma unroll
-          for (int pb = 0; pb < kPB; ++pb)
-            acc[rb][h][pb] = mfma16(as_bf16x8(f.a[rb]), as_bf16x8(f.b[h][pb]), acc[rb][h][pb]);
+        for (int cb = 0; cb < kCB; ++cb)
+          acc[rb][cb] = mfma16(as_bf16x8(f.a[rb]), as_bf16x8(f.b[cb]), acc[rb][cb]);
     };
     // the next half-step's LDS reads spread between this half-step's MFMAs
-    constexpr int kReads = kRB + 2 * kPB, kMfma = 2 * kRB * kPB;
+    constexpr int kReads = kRB + kCB, kMfma = kRB * kCB;
     constexpr int kEvery = kMfma / kReads;  // MFMAs after each read
     auto interleave = [&]() {
       if constexpr (kEvery == 0) return;  // fewer MFMAs than reads: the compiler's order
@@ -325,19 +320,17 @@ __global__ __launch_bounds__((4 + NPROD) * 64, 1) void pair_pc_kernel(PairGemmTi
       stage = next;
     }
 
-    // Stage the accumulators as fp32 rows in LDS: acc[rb][h][pb][i] is row
-    // BM/WM wm + 16 rb + 4 g4 + i, local pair kWP wn + 16 pb + l16, low (h = 0) or high.
+    // Stage the accumulators as fp32 rows in LDS: acc[rb][cb][i] is row
+    // BM/WM wm + 16 rb + 4 g4 + i, column kCols wn + 16 cb + l16.
     pg_barrier_lds();  // every LDS read done, every producer load landed
     float* staged = reinterpret_cast<float*>(smem);
 #pragma unroll
     for (int rb = 0; rb < kRB; ++rb)
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
-        float* row = staged + ((BM / WM) * wm + 16 * rb + 4 * g4 + i) * kEpStride + kWP * wn + l16;
+        float* row = staged + ((BM / WM) * wm + 16 * rb + 4 * g4 + i) * kEpStride + kCols * wn + l16;
 #pragma unroll
-        for (int h = 0; h < 2; ++h)
-#pragma unroll
-          for (int pb = 0; pb < kPB; ++pb) row[BP * h + 16 * pb] = acc[rb][h][pb][i];
+        for (int cb = 0; cb < kCB; ++cb) row[16 * cb] = acc[rb][cb][i];
       }
     if (tid < BM) reinterpret_cast<typename Ep::Row*>(smem + Sh::kEpMetaOff)[tid] = my_row;
     pg_barrier_lds();

@@ -25,9 +25,9 @@
 // tiles of another kernel, fdl_pair_gemm.h; see qkv_split):
 //  * more than 128 rows: 128 rows x 96 pairs, 4 stages of 40 KB (all of LDS). 512 rows give
 //    one tile per CU.
-//  * up to 128 rows (weight streaming, HBM-bound): 64 or 128 rows x 32 pairs (192 tiles at
-//    d_model 4096), 8 stages of 16 KB or 6 of 24 KB, so each workgroup keeps 5-7 weight
-//    steps in flight.
+//  * up to 128 rows (weight streaming, HBM-bound): 64 or 128 rows x 24 pairs (256 tiles at
+//    d_model 4096; 32 pairs beyond), 8 stages of 14 KB or 6 of 22 KB, so each workgroup keeps
+//    5-7 weight steps in flight.
 #include <algorithm>
 #include <atomic>
 #include <type_traits>
@@ -196,9 +196,8 @@ struct QkvSplit {
   int64_t wide, mid;
 };
 
-// Up to 128 rows the projection streams the weights (32-pair tiles, 192 workgroups, 6-8 stages:
-// 18.6 us at 40 rows, 23 us at 128; 128 x 32-pair tiles take 45 us at 192 rows against 36 us
-// for the 128 x 96-pair ones). Beyond, two shapes feed the MFMAs: a round of 256-row tiles (80
+// Up to 128 rows the projection streams the weights (24- or 32-pair tiles, 6-8 stages; 128 x
+// 32-pair tiles take 45 us at 192 rows against 36 us for the 128 x 96-pair ones). Beyond, two shapes feed the MFMAs: a round of 256-row tiles (80
 // us at d_model 4096, one workgroup per CU) covers as much as two rounds of 128-row tiles (47
 // us each), so whole rounds go to the 256-row tiles and a part of a round to what covers it
 // soonest: 512 rows to 128-row tiles (54 us; 256-row tiles fill half of the device and take
@@ -261,10 +260,10 @@ hipError_t qkv_launch(void (*kernel)(PairGemmTiles, RopeEp), int bm, int bp, int
                      3 * int64_t(args.n_heads) * kHalf, RopeEp{args}, stream);
 }
 
-template <int BM, int BP, int NPROD, int STAGES>
+template <int BM, int BP, int NPROD, int STAGES, int WM>
 hipError_t qkv_launch_pc(const QkvArgs& args, hipStream_t stream) {
-  return qkv_launch(pair_pc_kernel<RopeEp, BM, BP, NPROD, STAGES, 2>, BM, BP,
-                    PcShape<BM, BP, NPROD, STAGES, 2>::kThreads, args, stream);
+  return qkv_launch(pair_pc_kernel<RopeEp, BM, BP, NPROD, STAGES, WM>, BM, BP,
+                    PcShape<BM, BP, NPROD, STAGES, WM>::kThreads, args, stream);
 }
 
 }  // namespace
@@ -347,11 +346,18 @@ extern "C" int fdl_qkv_rope_cache(const void* x, const void* wq, const void* wk,
     FDL_HIP_CHECK(qkv_launch(pair_gemm_kernel<RopeEp>, kPgBM, kPgBP, kPgThreads,
                              qkv_rows(args, 0, split.wide), st));
   if (split.mid > 0)
-    FDL_HIP_CHECK((qkv_launch_pc<kPcBM, kPcBP, 4, 4>(qkv_rows(args, split.wide, split.mid), st)));
+    FDL_HIP_CHECK((qkv_launch_pc<kPcBM, kPcBP, 4, 4, 2>(qkv_rows(args, split.wide, split.mid), st)));
   if (rest > 0) {
     const QkvArgs tail = qkv_rows(args, split.wide + split.mid, rest);
-    FDL_HIP_CHECK((rest <= 64 ? qkv_launch_pc<64, 32, 4, 8>(tail, st)
-                              : qkv_launch_pc<128, 32, 4, 6>(tail, st)));
+    // 24-pair tiles while they are one round of workgroups (d_model 4096: all 256 CUs instead of
+    // the 192 that 32-pair tiles occupy), with two producers, which load as fast as more: cold
+    // weights, 40 rows 23.0 -> 21.5 us, 64 rows 25.0 -> 23.0, 100 rows 29.2 -> 28.3; d_model 2048,
+    // 64 rows 13.5 -> 12.6
+    const bool narrow = n_heads * 3 * kHalf / 24 <= pg_device_cus();
+    FDL_HIP_CHECK((rest <= 64 ? (narrow ? qkv_launch_pc<64, 24, 2, 8, 4>(tail, st)
+                                        : qkv_launch_pc<64, 32, 4, 8, 2>(tail, st))
+                              : (narrow ? qkv_launch_pc<128, 24, 2, 6, 4>(tail, st)
+                                        : qkv_launch_pc<128, 32, 4, 6, 2>(tail, st))));
   }
   return ok();
 }

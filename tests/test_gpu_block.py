@@ -163,7 +163,8 @@ def test_block_mlp_tail_split_k_ff_out_matches_single_product():
 
 @pytest.mark.parametrize("chunks", [1, 4])
 @pytest.mark.parametrize("rows,k,width", [
-    (1, 256, 96), (64, 4096, 12288), (65, 384, 12288), (17, 640, 192),  # weight-streaming tiles
+    # weight-streaming tiles of 24 (width up to 6144) and of 48 pairs
+    (1, 256, 96), (64, 4096, 12288), (65, 384, 12288), (17, 640, 192), (100, 256, 6144), (33, 256, 6240),
     (128, 256, 192), (129, 256, 96), (256, 512, 12288),                 # 128-row tiles
     (257, 256, 12288), (300, 384, 12384), (600, 512, 12288),            # 256-row tiles
 ])
