@@ -119,23 +119,27 @@ __global__ __launch_bounds__(kDirectThreads) void softmax_conf_direct_kernel(
 // ---- vocab from kTableVocab on
 //
 // What bounds the row: 126464 float64 exponentials by one workgroup are far more work than its
-// 253 KB of reads (64 us of the 70 us at 256 rows when each is computed), and a second read of
-// the row comes from the Infinity Cache. bf16 logits have few distinct values, so the
-// exponentials of the common ones are tabulated once per row in LDS (4096 per row instead of
-// 126464) and summed by look-up, and the row stays in registers between the passes: 256 rows
-// of 126464 70 -> 24 us, 32 rows 58 -> 20 us, 512 rows of 32000 31 -> 20 us. What is left is
-// mostly the look-ups (bank conflicts of random 8-byte reads). Below 16384 values the table
-// costs more than it saves (512 rows of 8192: 10 us computed, 14 us tabulated; of 16384: 17
-// and 17 us; one row of 16384: 10 and 8 us), so shorter rows keep the direct kernel.
+// 253 KB of reads (64 us of the 70 us at 256 rows when each is computed). bf16 logits have few
+// distinct values, so the exponentials of the common ones are tabulated once per row in LDS
+// (4096 per row instead of 126464) and summed by look-up. The table is of exp(x), not exp(x -
+// max): float64 holds it for |x| < 64 with the same relative precision, so a row whose maximum
+// lies there is read once, its maximum found and its sum formed as the values arrive (with a
+// table of exp(x - max) the look-ups began when the whole row had been read: 24.4 us at 256 rows
+// of 126464 against 19.6). Other rows take a second pass with a table of exp(x - max). Measured
+// (us), each exponential computed / tabulated: 256 rows of 126464 69.9 / 19.6, 32 rows 57.7 / 19.3,
+// 512 rows of 32000 30.9 / 20.1. What is left are the look-ups (random 8-byte LDS reads) and
+// their addresses: one row alone takes 18 us. Below 16384 values the table costs more than it
+// saves (512 rows of 8192: 10.0 computed, 14 tabulated; of 16384: 16.9 and 16.4), so shorter rows
+// keep the direct kernel.
 constexpr int64_t kTableVocab = 16384;
 
-// exp(x - m) of the bf16 values with |x| in [2^-10, 2^6) (16 exponents, both signs) from a
-// table of float64 values made once per row: a bf16 of those exponents is its sign, the low
-// 4 bits of its exponent and its 7 fraction bits. Values outside (also 0, NaN, infinities)
-// take exp() itself.
+// exp of the bf16 values with |x| in [2^-10, 2^6) (16 exponents, both signs) from a table of
+// float64 values: a bf16 of those exponents is its sign, the low 4 bits of its exponent and its
+// 7 fraction bits. Values outside (also 0, NaN, infinities) take exp() itself.
 constexpr uint32_t kTabMagLo = 117u << 7;  // bits of 2^-10
 constexpr uint32_t kTabMags = 16u << 7;
 constexpr int kTabSize = 2 * kTabMags;  // 4096 values, 32 KB
+constexpr float kTabLimit = 64.f;
 
 // whether all 8 values of v are in the table (the smallest and the largest magnitude bits, two
 // 16-bit halves at a time)
@@ -151,7 +155,7 @@ __device__ __forceinline__ bool in_table(u32x4 v) {
   return min(lo[0], lo[1]) >= kTabMagLo && max(hi[0], hi[1]) < kTabMagLo + kTabMags;
 }
 
-// sum of the table's exp(x_j - m) over the 8 values of v (any bits read inside the table)
+// sum of the table's values over the 8 values of v (any bits read inside the table)
 __device__ __forceinline__ double table_sum8(u32x4 v, const double* tab) {
   double s0 = 0.0, s1 = 0.0;
 #pragma unroll
@@ -173,10 +177,20 @@ __device__ __forceinline__ double exp_sum8(u32x4 v, double md) {
   return s;
 }
 
+// tab[i] = exp(x - ref) of the 4096 values
+__device__ __forceinline__ void make_table(double* tab, double ref) {
+#pragma unroll 1
+  for (int i = 0; i < kTabSize / kConfThreads; ++i) {
+    const uint32_t t = threadIdx.x + kConfThreads * i;
+    const uint32_t low = t & (kTabMags - 1);
+    // the magnitude of the range whose low 11 bits these are
+    const uint32_t mag = kTabMagLo + ((low - kTabMagLo) & (kTabMags - 1));
+    tab[t] = exp(static_cast<double>(bf2f(static_cast<uint16_t>(mag | (t / kTabMags) << 15))) - ref);
+  }
+}
+
 // vocab % 8 == 0 and 16-byte aligned rows (checked on the host). Thread t takes the 16-byte
-// chunks t, t + 1024, ..; with kChunks > 0 (vocab <= 8192 kChunks) they stay in registers, so
-// the row is read from memory once; with kChunks == 0 the second pass reads it again.
-template <int kChunks>
+// chunks t, t + 1024, ..
 __global__ __launch_bounds__(kConfThreads) void softmax_conf_kernel(
     const uint16_t* __restrict__ logits, int64_t vocab, const int64_t* __restrict__ token,
     double* __restrict__ prob, int64_t* __restrict__ arg) {
@@ -187,32 +201,55 @@ __global__ __launch_bounds__(kConfThreads) void softmax_conf_kernel(
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const uint16_t* x = logits + int64_t(blockIdx.x) * vocab;
   const int64_t n8 = vocab / 8;
+  const int n_own = static_cast<int>((n8 - tid + kConfThreads - 1) / kConfThreads);  // n8 >= 2048
+  auto chunk = [&](int i) { return ld16(x + 8 * (tid + int64_t(kConfThreads) * min(i, n_own - 1))); };
 
-  // the maximum (a NaN is never it; it makes the sum NaN)
-  u32x4 reg[kChunks > 0 ? kChunks : 1];
+  // One pass: the maximum, the first own chunk that holds it (a NaN is never the maximum; it
+  // makes the sum NaN) and the sum of exp(x - ref). kAhead chunks are in flight. Chunks with
+  // values outside the table wait in `rest` (the first 64): a wavefront would pay for every
+  // lane's one by one, and a row that takes a second pass need not sum them in the first.
+  constexpr int kAhead = 4;
   float m = -INFINITY;
-  auto max8 = [&](u32x4 v) {
+  int best = 0;
+  double s = 0.0;
+  uint64_t rest = 0;
+  auto pass = [&](double ref, u32x4 (&cur)[kAhead]) {
+    for (int i0 = 0; i0 < n_own; i0 += kAhead) {
+      u32x4 next[kAhead];
 #pragma unroll
-    for (int j = 0; j < 4; ++j) m = fmaxf(m, fmaxf(bf16_lo(v[j]), bf16_hi(v[j])));
-  };
-  if constexpr (kChunks > 0) {
+      for (int u = 0; u < kAhead; ++u) next[u] = chunk(i0 + kAhead + u);
 #pragma unroll
-    for (int i = 0; i < kChunks; ++i) {
-      const int64_t c = tid + int64_t(kConfThreads) * i;
-      reg[i] = ld16(x + 8 * min(c, n8 - 1));  // past the end: the last chunk, not summed
+      for (int u = 0; u < kAhead; ++u) {
+        if (i0 + u < n_own) {
+          const u32x4 v = cur[u];
+          float top = fmaxf(bf16_lo(v[0]), bf16_hi(v[0]));
+#pragma unroll
+          for (int j = 1; j < 4; ++j) top = fmaxf(top, fmaxf(bf16_lo(v[j]), bf16_hi(v[j])));
+          best = top > m ? i0 + u : best;
+          m = fmaxf(m, top);
+          if (in_table(v))
+            s += table_sum8(v, tab);
+          else if (i0 + u < 64)
+            rest |= uint64_t(1) << (i0 + u);
+          else
+            s += exp_sum8(v, ref);
+        }
+      }
+#pragma unroll
+      for (int u = 0; u < kAhead; ++u) cur[u] = next[u];
     }
-#pragma unroll
-    for (int i = 0; i < kChunks; ++i) max8(reg[i]);
-  } else {
-#pragma unroll 4
-    for (int64_t c = tid; c < n8; c += kConfThreads) max8(ld16(x + 8 * c));
-  }
-  // the chunks stay packed between the passes (no widened copies are carried over)
-  auto repack = [&]() {
-#pragma unroll
-    for (int i = 0; i < (kChunks > 0 ? kChunks : 0); ++i) asm volatile("" : "+v"(reg[i]));
   };
-  repack();
+  auto first_chunks = [&](u32x4 (&cur)[kAhead]) {
+#pragma unroll
+    for (int u = 0; u < kAhead; ++u) cur[u] = chunk(u);
+  };
+  u32x4 cur[kAhead];
+  first_chunks(cur);  // arrive while the table is made
+  make_table(tab, 0.0);
+  __syncthreads();
+  pass(0.0, cur);
+
+  // the row's maximum and its first index (only threads that hold it look)
   const float m_own = m;
 #pragma unroll
   for (int off = 32; off >= 1; off >>= 1) m = fmaxf(m, __shfl_xor(m, off));
@@ -222,73 +259,37 @@ __global__ __launch_bounds__(kConfThreads) void softmax_conf_kernel(
 #pragma unroll
   for (int w = 1; w < kConfWaves; ++w) m = fmaxf(m, s_m[w]);
   const double md = static_cast<double>(m);
-
-  // the table, and the first index of the maximum (only threads that hold it look)
-#pragma unroll 1
-  for (int i = 0; i < kTabSize / kConfThreads; ++i) {
-    const uint32_t t = tid + kConfThreads * i;
-    const uint32_t low = t & (kTabMags - 1);
-    // the magnitude of the range whose low 11 bits these are
-    const uint32_t mag = kTabMagLo + ((low - kTabMagLo) & (kTabMags - 1));
-    tab[t] = exp(static_cast<double>(bf2f(static_cast<uint16_t>(mag | (t / kTabMags) << 15))) - md);
-  }
   int64_t im = INT64_MAX;
   if (m_own == m) {
-    auto first8 = [&](u32x4 v, int64_t c) {
+    const u32x4 v = chunk(best);
+    const int64_t c = 8 * (tid + int64_t(kConfThreads) * best);
 #pragma unroll
-      for (int j = 3; j >= 0; --j) {
-        if (bf16_hi(v[j]) == m) im = min(im, 8 * c + 2 * j + 1);
-        if (bf16_lo(v[j]) == m) im = min(im, 8 * c + 2 * j);
-      }
-    };
-    if constexpr (kChunks > 0) {
-      int hit = 0;  // the first chunk with the maximum
-#pragma unroll
-      for (int i = kChunks - 1; i >= 0; --i) {
-        float top = -INFINITY;
-#pragma unroll
-        for (int j = 0; j < 4; ++j) top = fmaxf(top, fmaxf(bf16_lo(reg[i][j]), bf16_hi(reg[i][j])));
-        hit = top == m ? i : hit;
-      }
-      const int64_t c = min(tid + int64_t(kConfThreads) * hit, n8 - 1);
-      first8(ld16(x + 8 * c), c);
-    } else {
-      for (int64_t c = tid; c < n8; c += kConfThreads) first8(ld16(x + 8 * c), c);
+    for (int j = 3; j >= 0; --j) {
+      if (bf16_hi(v[j]) == m) im = c + 2 * j + 1;
+      if (bf16_lo(v[j]) == m) im = c + 2 * j;
     }
   }
-#pragma unroll
-  for (int off = 32; off >= 1; off >>= 1) im = min(im, __shfl_xor(im, off));
-  if (lane == 0) s_i[wave] = im;
-  __syncthreads();
-
-  // float64 sum of exp(x - m): per-thread partials, then a fixed reduction tree
-  repack();
-  double s = 0.0;
-  if constexpr (kChunks > 0) {
-    uint32_t rest = 0;  // this thread's chunks that are not all in the table
-#pragma unroll
-    for (int i = 0; i < kChunks; ++i) {
-      if (tid + int64_t(kConfThreads) * i < n8) {
-        if (in_table(reg[i]))
-          s += table_sum8(reg[i], tab);
-        else
-          rest |= 1u << i;
-      }
-      if (i % 2) __builtin_amdgcn_sched_barrier(0);  // 16 look-ups in flight
-    }
-    for (; rest; rest &= rest - 1) {
-      const int64_t c = tid + int64_t(kConfThreads) * __builtin_ctz(rest);
-      s += exp_sum8(ld16(x + 8 * c), md);
-    }
-  } else {
-    for (int64_t c = tid; c < n8; c += kConfThreads) {
-      const u32x4 v = ld16(x + 8 * c);
-      s += in_table(v) ? table_sum8(v, tab) : exp_sum8(v, md);
-    }
+  // a maximum outside the table's range: sums of exp(x) may overflow or vanish
+  const bool ranged = m >= -kTabLimit && m < kTabLimit;
+  if (!ranged) {
+    make_table(tab, md);  // every look-up came before the barrier above
+    __syncthreads();
+    s = 0.0;
+    rest = 0;
+    first_chunks(cur);
+    pass(md, cur);
   }
+  for (; rest; rest &= rest - 1)
+    s += exp_sum8(chunk(__builtin_ctzll(rest)), ranged ? 0.0 : md);
 #pragma unroll
-  for (int off = 32; off >= 1; off >>= 1) s += __shfl_xor(s, off);
-  if (lane == 0) s_sum[wave] = s;
+  for (int off = 32; off >= 1; off >>= 1) {
+    s += __shfl_xor(s, off);
+    im = min(im, __shfl_xor(im, off));
+  }
+  if (lane == 0) {
+    s_sum[wave] = s;
+    s_i[wave] = im;
+  }
   __syncthreads();
   if (tid == 0) {
     double sum = s_sum[0];
@@ -298,6 +299,7 @@ __global__ __launch_bounds__(kConfThreads) void softmax_conf_kernel(
       sum += s_sum[w];
       im = min(im, s_i[w]);
     }
+    if (ranged) sum *= exp(-md);  // sum of exp(x - m)
     double p;
     if (token) {
       const int64_t t = token[blockIdx.x];
@@ -328,12 +330,8 @@ extern "C" int fdl_softmax_confidence(const void* logits, int64_t n_rows, int64_
   FDL_REQUIRE_PTR(logits);
   FDL_REQUIRE_PTR(prob);
   FDL_REQUIRE_ALIGNED(logits, 16);
-  constexpr int64_t per_chunk = int64_t(8) * kConfThreads;  // values per chunk of a workgroup
   const bool direct = vocab < kTableVocab;
-  auto* kernel = direct                    ? softmax_conf_direct_kernel
-                 : vocab <= 4 * per_chunk  ? softmax_conf_kernel<4>
-                 : vocab <= 16 * per_chunk ? softmax_conf_kernel<16>
-                                           : softmax_conf_kernel<0>;
+  auto* kernel = direct ? softmax_conf_direct_kernel : softmax_conf_kernel;
   hipLaunchKernelGGL(kernel, dim3(static_cast<unsigned>(n_rows)),
                      dim3(direct ? kDirectThreads : kConfThreads), 0,
                      static_cast<hipStream_t>(stream), static_cast<const uint16_t*>(logits), vocab,

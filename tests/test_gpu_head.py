@@ -63,23 +63,27 @@ def test_softmax_confidence_non_finite_rows_match_torch():
     np.testing.assert_allclose(got_p[3:].numpy(), ref_p[3:].numpy(), rtol=1e-12)
 
 
-@pytest.mark.parametrize("vocab", [16376, 16384, 32768, 32776, 131072, 131080])
+@pytest.mark.parametrize("vocab", [16376, 16384, 16392, 24568, 32776, 131080, 532488])
 @pytest.mark.parametrize("token", [False, True])
 def test_softmax_confidence_kernel_edges(vocab, token):
-    """The vocabulary sizes at which another kernel takes over (direct, tabulated with the row
-    in registers, tabulated with the row read twice), on rows that hold the edges of the
-    tabulated range of magnitudes ([2^-10, 2^6)) and values outside it: zeros, denormals,
-    -inf, large ones. The terms are the reference's to an ulp or two of float64 and only the
-    order of up to 131080 positive terms differs: 1e-12 relative."""
+    """Vocabulary sizes around the one at which the tabulated kernel takes over, at its chunk
+    counts' edges and past the 64 chunks of a thread that it can put off, on rows that hold the
+    edges of the tabulated range of magnitudes ([2^-10, 2^6)) and values outside it (zeros,
+    denormals, -inf, large ones), and rows whose maximum lies outside it (a second pass). The
+    terms are the reference's to an ulp or two of float64 and only the order of up to 532488
+    positive terms differs: 1e-12 relative."""
     gen = torch.Generator().manual_seed(vocab)
-    x = (torch.randn(4, vocab, generator=gen) * 3.0).to(torch.bfloat16)
+    x = (torch.randn(7, vocab, generator=gen) * 3.0).to(torch.bfloat16)
     edge = torch.tensor([0.0, -0.0, 2.0**-10, -2.0**-10, 2.0**-10 * (1 - 2.0**-8), 1e-40, -1e-40,
                          63.75, -63.75, -64.0, -700.0, -3e38, float("-inf")]).to(torch.bfloat16)
     x[1, 40:40 + len(edge)] = edge
     x[1, vocab - len(edge):] = edge
     x[2] = (x[2].float() * 40.0).to(torch.bfloat16)  # most values past the table
     x[3] = 0.0                                         # nothing in the table, all tied
-    tok = torch.tensor([vocab - 1, 41, int(x[2].argmax()), vocab])
+    x[4] = (x[4].float() - 400.0).to(torch.bfloat16)  # sums of exp(x) vanish
+    x[5, vocab - 1] = 900.0                            # exp(x) overflows
+    x[6, 3] = 64.0                                     # the first maximum outside the range
+    tok = torch.tensor([vocab - 1, 41, int(x[2].argmax()), vocab, 9, vocab - 1, 3])
     p = F.softmax(x.double(), dim=-1)
     ref_p, ref_i = torch.max(p, dim=-1)
     if token:
