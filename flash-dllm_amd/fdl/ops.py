@@ -476,8 +476,18 @@ def silu_mul(gate: torch.Tensor, up: torch.Tensor, out: torch.Tensor | None = No
 def gate_up_silu_pays(rows: int, width: int, device: torch.device) -> bool:
     """Whether gate_up_silu is faster than one library product over both weights and silu_mul:
     while its 128-row tiles fit one round of workgroups (width 12288: up to 256 rows; 64 rows
-    50 -> 37 us, 256 rows 67 -> 61 us; 640 rows 132 -> 158 us)."""
-    return 0 < rows and -(-rows // 128) * (width // 96) <= _cus(device)
+    50 -> 37 us, 256 rows 67 -> 61 us), and where its 256-row tiles make one to three whole rounds
+    and are at least 25/32 full of rows (400-512 rows 98-103 -> 92-95 us, 1024 190 -> 180, 1536
+    277 -> 266; against it 384 rows 87 / 93 us, 640 rows 132 / 158, 1280 rows 220 / 246, 2048 rows
+    316 / 349)."""
+    if rows <= 0:
+        return False
+    cus, n_tiles = _cus(device), width // 96
+    if -(-rows // 128) * n_tiles <= cus:
+        return True
+    m_tiles = -(-rows // 256)
+    return (m_tiles * n_tiles % cus == 0 and m_tiles * n_tiles <= 3 * cus
+            and rows >= 200 * m_tiles)
 
 
 def gate_up_silu(x: torch.Tensor, w_gate: torch.Tensor, w_up: torch.Tensor,
