@@ -1,12 +1,16 @@
-// GEMM over pairs of weight rows (gfx950, bf16 MFMA, fp32 sums), for many input rows:
+// GEMM over pairs of weight rows (gfx950, bf16 MFMA, fp32 sums):
 //   lo[r][p] = x_r . w_lo(p),  hi[r][p] = x_r . w_hi(p)        (reduction length K)
 // handed to an epilogue that sees both members of a pair. The Q/K/V projection pairs the two
-// columns that RoPE rotates together.
+// columns that RoPE rotates together, the MLP a column's gate and up rows.
 //
-// Tile: 256 rows x 96 pairs (192 weight rows), eight wavefronts (4 x 2, each 64 rows x 48
-// pairs, two per SIMD) that load, read LDS and multiply alike.
+// pair_pc_kernel: up to 128 rows per tile, wavefronts in two roles (producers that only load,
+// consumers that only read LDS and multiply), a deep ring of stages; also the weight-streaming
+// kernel of few rows.
 //
-// What bounds it: the L2 -> LDS path moves 26-36 B/clk per CU with every CU loading, and a tile
+// pair_gemm_kernel: 256 rows x 96 pairs (192 weight rows) per tile, eight wavefronts (4 x 2, each
+// 64 rows x 48 pairs, two per SIMD) that load, read LDS and multiply alike.
+//
+// What bounds the latter: the L2 -> LDS path moves 26-36 B/clk per CU with every CU loading, and a tile
 // of m x n needs 128 (m + n) bytes per 64-deep step of m n / 32 MFMA clocks. 256 x 192 needs 36
 // B/clk at the full MFMA rate, the 128 x 192 tile of the smaller shape 53: that one spends its
 // time on loads. Both operands are requested two steps ahead (three weight stages: weights may

@@ -20,9 +20,10 @@ half runs on the hand-written gfx950 kernels behind the C ABI (include/fdl.h):
     fdl_verify_attention     cache keys through key_pos_flat + in-block keys under attn_mask
 
 The RMSLayerNorms and the SiLU gate run on fused HIP kernels (fdl_rms_norm, with the
-attention residual add folded into ff_norm's pass, and fdl_silu_mul); the projections of
-the MLP half (attn_out, ff_proj, up_proj, ff_out; :618-636) are plain library GEMMs through
-torch, as in the reference. Norm or activation modules of other kinds run as the modules
+attention residual add folded into ff_norm's pass, and fdl_silu_mul). The products of the MLP
+half (attn_out, ff_proj, up_proj, ff_out; :618-636) are hand-written kernels where they are the
+faster way, mostly for few rows (fdl_gate_up_silu, fdl_linear_partials), and plain library GEMMs
+through torch otherwise. Norm, activation or attn_out modules of other kinds run as the modules
 themselves.
 
 positions = [query_pos_flat, key_pos_flat, [sin, cos], info, attn_scores, attn_mask]
