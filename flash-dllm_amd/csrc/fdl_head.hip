@@ -9,8 +9,11 @@
 //   probability of token t = exp(x_t - m) / s.
 // A row with a NaN, a +inf or only -inf logits has a softmax of NaNs: probability NaN and
 // index 0, as torch.max returns for it.
-// bf16 -> float -> double is exact, so every term is the float64 softmax term; only the
-// order of the float64 sum differs from torch's reduction.
+// bf16 -> float -> double is exact. Of few values (below kTableVocab) and where |m| is large,
+// the terms are the float64 softmax's and only the order of the float64 sum differs from
+// torch's reduction; otherwise s = sum_j exp(x_j) / exp(m), whose terms differ by an ulp or
+// two. s >= 1 either way, so no probability exceeds 1, and a row whose maximum holds everything
+// has exactly 1.
 #include <stdint.h>
 
 #include "fdl_device.h"
@@ -299,7 +302,10 @@ __global__ __launch_bounds__(kConfThreads) void softmax_conf_kernel(
       sum += s_sum[w];
       im = min(im, s_i[w]);
     }
-    if (ranged) sum *= exp(-md);  // sum of exp(x - m)
+    // The sum of exp(x - m). Divided by exp(m), which is one of its terms: times exp(-m), a row
+    // whose maximum holds everything would not give exactly 1 (exp(m) exp(-m) is above or below
+    // 1 for a third of the maxima), and its probability could exceed 1.
+    if (ranged) sum /= exp(md);
     double p;
     if (token) {
       const int64_t t = token[blockIdx.x];

@@ -1,8 +1,8 @@
 """LM-head confidence (fdl_softmax_confidence) against the float64 torch code it replaces
 (generate.py:218, :320, :337): max(softmax(logits.double())) and its index, and the
 softmax probability of a given token. The reference is torch's float64 softmax on the CPU:
-the float64 terms are identical and only the order of the sum differs, so probabilities
-agree to ~1e-13 relative and indices exactly. (torch's float64 softmax kernel on this ROCm
+the float64 terms are identical, or (many values) exp(x) in place of exp(x - m), and the order
+of the sum differs, so probabilities agree to ~1e-13 relative and indices exactly. (torch's float64 softmax kernel on this ROCm
 build is itself ~1e-9 off the CPU result, so it is not the reference here.)"""
 import numpy as np
 import pytest
@@ -92,3 +92,27 @@ def test_softmax_confidence_kernel_edges(vocab, token):
     prob, arg = ops.softmax_confidence(x.to(DEV), tok.to(DEV) if token else None)
     torch.testing.assert_close(prob.cpu(), ref_p, rtol=1e-12, atol=0)
     assert torch.equal(arg.cpu(), ref_i)
+
+
+@pytest.mark.parametrize("vocab", [1024, 16384])
+def test_softmax_confidence_of_a_certain_row_is_exactly_one(vocab):
+    """A row whose maximum holds everything (the rest at least 69 below it: less than 2^-53 of the
+    sum) has probability 1.0, and one whose maximum is tied 0.5, as float64 softmax gives: for
+    every magnitude from 2^-11 to 2^7 in bf16 and both signs (the tabulated maxima and those
+    around them), so such rows stay tied with each other and pass a threshold of 1."""
+    bits = torch.arange(116 << 7, 134 << 7)
+    m = torch.cat((bits, bits | 0x8000)).to(torch.int16).view(torch.bfloat16).to(DEV)
+    gen = torch.Generator(device=DEV).manual_seed(vocab)
+    for top in m.split(1536):
+        rows = len(top)
+        low = torch.rand((rows, vocab), generator=gen, device=DEV) * 6.0 + 70.0
+        x = (top.float()[:, None] - low).to(torch.bfloat16)
+        at = torch.randint(0, vocab, (rows,), generator=gen, device=DEV)
+        r = torch.arange(rows, device=DEV)
+        x[r, at] = top
+        for token in (None, at):
+            prob, arg = ops.softmax_confidence(x, token)
+            assert (prob == 1.0).all(), (prob.min(), prob.max())
+            assert torch.equal(arg, at)
+        x[r, (at + 7) % vocab] = top
+        assert (ops.softmax_confidence(x)[0] == 0.5).all()
