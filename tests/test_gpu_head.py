@@ -45,22 +45,36 @@ def test_softmax_confidence_token_probability():
     torch.testing.assert_close(prob.cpu(), ref, rtol=1e-12, atol=1e-300)
 
 
-def test_softmax_confidence_non_finite_rows_match_torch():
+@pytest.mark.parametrize("vocab", [1024, 16384, 126464, 532488])
+@pytest.mark.parametrize("token", [False, True])
+def test_softmax_confidence_non_finite_rows_match_torch(vocab, token):
     """Rows of all -inf, with a NaN, with a +inf, and with the maximum tied at several
     places: the probability and index are torch.max(softmax(float64)) of the row (NaN and
-    index 0 for the rows whose softmax is NaN; the first index of a tie)."""
-    vocab = 1024
-    x = torch.randn((5, vocab), generator=torch.Generator().manual_seed(3)).to(torch.bfloat16)
+    index 0 for the rows whose softmax is NaN; the first index of a tie). NaN and +inf stand in a
+    row's first and last values (532488: past the chunks that the tabulated kernel can put off),
+    and the NaN also in a row whose maximum forces a second pass."""
+    x = torch.randn((9, vocab), generator=torch.Generator().manual_seed(3)).to(torch.bfloat16)
     x[0] = float("-inf")
     x[1, 300] = float("nan")
     x[2, 700] = float("inf")
-    x[3, 10] = x[3, 500] = x[3, 900] = 8.0  # tied maximum
-    prob, arg = ops.softmax_confidence(x.to(DEV))
-    ref_p, ref_i = torch.max(torch.softmax(x.double(), dim=-1), dim=-1)
+    x[3, vocab - 2] = float("nan")
+    x[4, vocab - 2] = float("inf")
+    x[5, 300], x[5, 20] = float("nan"), 500.0
+    x[6, vocab - 2], x[6, 20] = float("nan"), -float("inf")
+    x[7, 10] = x[7, 500] = x[7, 900] = 8.0  # tied maximum
+    x[8] = float("-inf")
+    x[8, 600] = -3.0                        # one value only
+    tok = torch.tensor([5, 300, 700, 9, 9, 20, 3, 500, 600])
+    prob, arg = ops.softmax_confidence(x.to(DEV), tok.to(DEV) if token else None)
+    p = torch.softmax(x.double(), dim=-1)
+    ref_p, ref_i = torch.max(p, dim=-1)
+    if token:
+        ref_p = p.gather(1, tok[:, None]).view(-1)
     got_p, got_i = prob.cpu(), arg.cpu()
     assert torch.equal(got_i, ref_i), (got_i, ref_i)
-    assert torch.isnan(got_p[:3]).all() and torch.isnan(ref_p[:3]).all()
-    np.testing.assert_allclose(got_p[3:].numpy(), ref_p[3:].numpy(), rtol=1e-12)
+    assert torch.isnan(got_p[:7]).all() and torch.isnan(ref_p[:7]).all()
+    np.testing.assert_allclose(got_p[7:].numpy(), ref_p[7:].numpy(), rtol=1e-12)
+    assert got_p[8] == 1.0
 
 
 @pytest.mark.parametrize("vocab", [16376, 16384, 16392, 24568, 32776, 131080, 532488])
