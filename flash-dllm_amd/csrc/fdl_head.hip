@@ -128,9 +128,12 @@ __global__ __launch_bounds__(kDirectThreads) void softmax_conf_direct_kernel(
 // max): float64 holds it for |x| < 64 with the same relative precision, so a row whose maximum
 // lies there is read once, its maximum found and its sum formed as the values arrive (with a
 // table of exp(x - max) the look-ups began when the whole row had been read: 24.4 us at 256 rows
-// of 126464 against 19.6). Other rows take a second pass with a table of exp(x - max). Measured
-// (us), each exponential computed / tabulated: 256 rows of 126464 69.9 / 19.6, 32 rows 57.7 / 19.3,
-// 512 rows of 32000 30.9 / 20.1. What is left are the look-ups (random 8-byte LDS reads) and
+// of 126464 against 19.6). Other rows take a second pass that computes every exponential: their
+// values mostly lie outside the table as well (a second table, of exp(x - max), took 51.7 us
+// against 43.0 at 256 x 126464 N(0, 200^2) values, 12.2 against 9.7 at 32 x 16384 N(0, 40^2)).
+// Measured (us), each exponential computed / tabulated: 256 rows of 126464 69.9 / 19.6, 32 rows
+// 57.7 / 19.3, 512 rows of 32000 30.9 / 20.1; of a second pass: 256 rows of 126464 70.0 / 43.0,
+// of 32000 16.5 / 15.3, of 16384 10.0 / 10.4, the one place that loses. What is left are the look-ups (random 8-byte LDS reads) and
 // their addresses: one row alone takes 18 us. Below 16384 values the table costs more than it
 // saves (512 rows of 8192: 10.0 computed, 14 tabulated; of 16384: 16.9 and 16.4), so shorter rows
 // keep the direct kernel.
@@ -180,15 +183,15 @@ __device__ __forceinline__ double exp_sum8(u32x4 v, double md) {
   return s;
 }
 
-// tab[i] = exp(x - ref) of the 4096 values
-__device__ __forceinline__ void make_table(double* tab, double ref) {
+// tab[i] = exp(x) of the 4096 values
+__device__ __forceinline__ void make_table(double* tab) {
 #pragma unroll 1
   for (int i = 0; i < kTabSize / kConfThreads; ++i) {
     const uint32_t t = threadIdx.x + kConfThreads * i;
     const uint32_t low = t & (kTabMags - 1);
     // the magnitude of the range whose low 11 bits these are
     const uint32_t mag = kTabMagLo + ((low - kTabMagLo) & (kTabMags - 1));
-    tab[t] = exp(static_cast<double>(bf2f(static_cast<uint16_t>(mag | (t / kTabMags) << 15))) - ref);
+    tab[t] = exp(static_cast<double>(bf2f(static_cast<uint16_t>(mag | (t / kTabMags) << 15))));
   }
 }
 
@@ -207,50 +210,45 @@ __global__ __launch_bounds__(kConfThreads) void softmax_conf_kernel(
   const int n_own = static_cast<int>((n8 - tid + kConfThreads - 1) / kConfThreads);  // n8 >= 2048
   auto chunk = [&](int i) { return ld16(x + 8 * (tid + int64_t(kConfThreads) * min(i, n_own - 1))); };
 
-  // One pass: the maximum, the first own chunk that holds it (a NaN is never the maximum; it
-  // makes the sum NaN) and the sum of exp(x - ref). kAhead chunks are in flight. Chunks with
-  // values outside the table wait in `rest` (the first 64): a wavefront would pay for every
-  // lane's one by one, and a row that takes a second pass need not sum them in the first.
   constexpr int kAhead = 4;
+  u32x4 cur[kAhead];
+#pragma unroll
+  for (int u = 0; u < kAhead; ++u) cur[u] = chunk(u);  // arrive while the table is made
+  make_table(tab);
+  __syncthreads();
+
+  // One pass: the maximum, the first own chunk that holds it (a NaN is never the maximum; it
+  // makes the sum NaN) and the sum of exp(x). kAhead chunks are in flight. Chunks with values
+  // outside the table wait in `rest` (the first 64): a wavefront would pay for every lane's one
+  // by one, and a row that takes a second pass need not sum them in the first.
   float m = -INFINITY;
   int best = 0;
   double s = 0.0;
   uint64_t rest = 0;
-  auto pass = [&](double ref, u32x4 (&cur)[kAhead]) {
-    for (int i0 = 0; i0 < n_own; i0 += kAhead) {
-      u32x4 next[kAhead];
+  for (int i0 = 0; i0 < n_own; i0 += kAhead) {
+    u32x4 next[kAhead];
 #pragma unroll
-      for (int u = 0; u < kAhead; ++u) next[u] = chunk(i0 + kAhead + u);
+    for (int u = 0; u < kAhead; ++u) next[u] = chunk(i0 + kAhead + u);
 #pragma unroll
-      for (int u = 0; u < kAhead; ++u) {
-        if (i0 + u < n_own) {
-          const u32x4 v = cur[u];
-          float top = fmaxf(bf16_lo(v[0]), bf16_hi(v[0]));
+    for (int u = 0; u < kAhead; ++u) {
+      if (i0 + u < n_own) {
+        const u32x4 v = cur[u];
+        float top = fmaxf(bf16_lo(v[0]), bf16_hi(v[0]));
 #pragma unroll
-          for (int j = 1; j < 4; ++j) top = fmaxf(top, fmaxf(bf16_lo(v[j]), bf16_hi(v[j])));
-          best = top > m ? i0 + u : best;
-          m = fmaxf(m, top);
-          if (in_table(v))
-            s += table_sum8(v, tab);
-          else if (i0 + u < 64)
-            rest |= uint64_t(1) << (i0 + u);
-          else
-            s += exp_sum8(v, ref);
-        }
+        for (int j = 1; j < 4; ++j) top = fmaxf(top, fmaxf(bf16_lo(v[j]), bf16_hi(v[j])));
+        best = top > m ? i0 + u : best;
+        m = fmaxf(m, top);
+        if (in_table(v))
+          s += table_sum8(v, tab);
+        else if (i0 + u < 64)
+          rest |= uint64_t(1) << (i0 + u);
+        else
+          s += exp_sum8(v, 0.0);
       }
-#pragma unroll
-      for (int u = 0; u < kAhead; ++u) cur[u] = next[u];
     }
-  };
-  auto first_chunks = [&](u32x4 (&cur)[kAhead]) {
 #pragma unroll
-    for (int u = 0; u < kAhead; ++u) cur[u] = chunk(u);
-  };
-  u32x4 cur[kAhead];
-  first_chunks(cur);  // arrive while the table is made
-  make_table(tab, 0.0);
-  __syncthreads();
-  pass(0.0, cur);
+    for (int u = 0; u < kAhead; ++u) cur[u] = next[u];
+  }
 
   // the row's maximum and its first index (only threads that hold it look)
   const float m_own = m;
@@ -275,15 +273,11 @@ __global__ __launch_bounds__(kConfThreads) void softmax_conf_kernel(
   // a maximum outside the table's range: sums of exp(x) may overflow or vanish
   const bool ranged = m >= -kTabLimit && m < kTabLimit;
   if (!ranged) {
-    make_table(tab, md);  // every look-up came before the barrier above
-    __syncthreads();
     s = 0.0;
-    rest = 0;
-    first_chunks(cur);
-    pass(md, cur);
+    for (int i = 0; i < n_own; ++i) s += exp_sum8(chunk(i), md);
+  } else {
+    for (; rest; rest &= rest - 1) s += exp_sum8(chunk(__builtin_ctzll(rest)), 0.0);
   }
-  for (; rest; rest &= rest - 1)
-    s += exp_sum8(chunk(__builtin_ctzll(rest)), ranged ? 0.0 : md);
 #pragma unroll
   for (int off = 32; off >= 1; off >>= 1) {
     s += __shfl_xor(s, off);
