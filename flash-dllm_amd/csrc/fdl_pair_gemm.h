@@ -56,7 +56,23 @@ struct PairGemmTiles {
   int k;        // reduction length of a workgroup (256-row tiles: a multiple of 128, at least 256)
   int n_mtiles, n_ntiles;
   int ld;       // row stride of x; the weight rows' is the epilogue's business
+  int start_mul;  // see pg_start
 };
+
+// The reduction step that the tile of pairs p0 .. starts its walk with (it wraps around). When all
+// workgroups read the same 128 bytes of their weight rows (a power of two apart) at a time, the
+// reads crowd on few HBM channels; cold weights, all in step / started apart: gate and up at 64
+// rows (201 MB) 46.8 / 36.9 us, at 128 rows 50.9 / 43.4, the 40-row projection (101 MB) 24.1 /
+// 22.1. The pairs are cut into groups of kPgStartPairs, a multiple of every tile's width, and the
+// groups spread over kPgStarts even places (8 places: 128 rows of gate and up 45.4 us; 32 or 64
+// no better than 16). The place depends on the pair and the number of pairs alone, so a row's
+// sums are added in the same order, and are the same bits, whatever the number of rows and the
+// tile. Launches of many row blocks gain nothing from it and lose nothing (6842 rows of the
+// projection 544 / 547 us).
+constexpr int kPgStartPairs = 96, kPgStarts = 16;
+__device__ __forceinline__ int pg_start(const PairGemmTiles& t, int p0, int nk) {
+  return ((p0 / kPgStartPairs * t.start_mul) >> 16) * nk / kPgStarts;
+}
 
 // 16 bytes per lane from global memory into LDS at lds + 16 * lane (lds wavefront-uniform),
 // issued where the compiler does not see it: it would otherwise wait for every load in flight
@@ -219,13 +235,7 @@ __global__ __launch_bounds__((4 + NPROD) * 64, 1) void pair_pc_kernel(PairGemmTi
       }
       dst_off[i] = 1024 * q;
     }
-    // With one row block every workgroup reads weights of its own, and starts its walk over the
-    // reduction at its own place: when all of them read the same 128 bytes of their rows (a
-    // power of two apart) at a time, the reads crowd on few HBM channels. Cold weights: gate and
-    // up at 64 rows (201 MB) 46.8 -> 37.1 us, the 40-row projection (101 MB) 24.1 -> 22.3 us,
-    // 128 rows of gate and up 50.9 -> 45.3 us. Row blocks that share weights keep in step (a
-    // start per tile or per XCD gained nothing at 512 to 6842 rows).
-    const int rot = t.n_mtiles == 1 ? static_cast<int>(int64_t(nt) * nk / t.n_ntiles) : 0;
+    const int rot = pg_start(t, BP * nt, nk);
     // Requests step kt (< nk) into `stage`. No step past the end is requested: the tail of the
     // loop waits for fewer steps instead (re-reading the last step there, to keep one wait
     // count, cost 1.3% at 512 rows).
@@ -398,7 +408,9 @@ __global__ __launch_bounds__(kPgThreads, 1) void pair_gemm_kernel(PairGemmTiles 
   // 8 q + lane / 8, LDS chunk lane % 8, which holds the row's chunk (lane % 8) ^ ((row >> 1) & 7):
   // two 128-byte rows share one 256-byte bank line, so 16 consecutive rows read at one chunk
   // land on 16 distinct 4-bank groups.
-  const uint16_t* abase = t.x + m0 * t.k;  // the next step to load
+  const int start = pg_start(t, kPgBP * nt, nk);
+  const uint16_t* abase = t.x + m0 * t.k + start * kPgKT;  // the next step to load
+  int to_wrap = nk - 1 - start;  // steps to load before the walk goes back to the first
   const int last = static_cast<int>(min(t.n_rows - m0, int64_t(kPgBM)) - 1);
   uint32_t aoff[kPgALoads];         // this lane's row and chunk, bytes from abase
   const uint16_t* bsrc[kPgBLoads];  // the next step to load
@@ -413,7 +425,7 @@ __global__ __launch_bounds__(kPgThreads, 1) void pair_gemm_kernel(PairGemmTiles 
     const int row = 8 * (8 * l + wave) + (lane >> 3);
     const int c = (lane & 7) ^ ((row >> 1) & 7);
     const int hi = row / kPgBP;
-    bsrc[l] = ep.wrow(kPgBP * nt + (row - hi * kPgBP), hi) + 8 * c;
+    bsrc[l] = ep.wrow(kPgBP * nt + (row - hi * kPgBP), hi) + start * kPgKT + 8 * c;
   }
   const uint32_t lds0 = static_cast<uint32_t>(reinterpret_cast<size_t>((PgLds)smem));
   const uint32_t a_lds = __builtin_amdgcn_readfirstlane(lds0 + 1024 * wave);
@@ -422,9 +434,11 @@ __global__ __launch_bounds__(kPgThreads, 1) void pair_gemm_kernel(PairGemmTiles 
     pg_dma16(abase, aoff[l],
              __builtin_amdgcn_readfirstlane(a_lds + uint32_t(stage * kPgABytes + 8192 * l)));
   };
+  int advance = 0;  // elements from the step that is being loaded to the next one
+  auto next_step = [&]() { advance = to_wrap-- == 0 ? kPgKT - t.k : kPgKT; };
   auto load_b = [&](int stage, int l) {
     pg_dma16(bsrc[l], __builtin_amdgcn_readfirstlane(b_lds + uint32_t(stage * kPgBBytes + 8192 * l)));
-    bsrc[l] += kPgKT;
+    bsrc[l] += advance;
   };
   u32x4 fa[2][kRB], fb[2][2 * kPB];
   f32x4 acc[kRB][2 * kPB];  // [row block][kPB hi + pair block]
@@ -449,9 +463,10 @@ __global__ __launch_bounds__(kPgThreads, 1) void pair_gemm_kernel(PairGemmTiles 
   // steps 0 and 1, in the order in which they are waited for
 #pragma unroll
   for (int s = 0; s < 2; ++s) {
+    next_step();
 #pragma unroll
     for (int l = 0; l < kPgALoads; ++l) load_a(s, l);
-    abase += kPgKT;
+    abase += advance;
 #pragma unroll
     for (int l = 0; l < kPgBLoads; ++l) load_b(s, l);
   }
@@ -478,6 +493,7 @@ __global__ __launch_bounds__(kPgThreads, 1) void pair_gemm_kernel(PairGemmTiles 
     const int bs2 = bs1 == kPgBStages - 1 ? 0 : bs1 + 1;
     const uint32_t a1 = (fa_off + as * kPgABytes) ^ 64, b1 = (fb_off + bs * kPgBBytes) ^ 64;
     const uint32_t a0 = fa_off + (as ^ 1) * kPgABytes, b0 = fb_off + bs1 * kPgBBytes;
+    if (kLoad) next_step();
 #pragma unroll
     for (int rb = 0; rb < kRB; ++rb) {
       if (kLoad && rb < kPgBLoads) load_b(bs2, rb);
@@ -507,7 +523,7 @@ __global__ __launch_bounds__(kPgThreads, 1) void pair_gemm_kernel(PairGemmTiles 
       mma(1, rb);
       __builtin_amdgcn_sched_barrier(0);
     }
-    if (kLoad) abase += kPgKT;
+    if (kLoad) abase += advance;
     bs = bs1;
   };
   constexpr std::true_type yes{};
@@ -575,8 +591,10 @@ hipError_t pair_launch(void (*kernel)(PairGemmTiles, Ep), int bm, int bp, int th
                        hipStream_t stream, int64_t n_split = 1) {
   const int64_t n_mtiles = (n_rows + bm - 1) / bm, n_ntiles = n_pairs / bp;
   if (n_mtiles * n_ntiles >= (int64_t(1) << 31)) return hipErrorInvalidValue;
+  const int64_t groups = (n_pairs + kPgStartPairs - 1) / kPgStartPairs;
   const PairGemmTiles t = {x, n_rows, static_cast<int>(k / n_split), static_cast<int>(n_mtiles),
-                           static_cast<int>(n_ntiles), static_cast<int>(k)};
+                           static_cast<int>(n_ntiles), static_cast<int>(k),
+                           static_cast<int>((kPgStarts << 16) / groups)};
   hipLaunchKernelGGL(kernel,
                      dim3(static_cast<unsigned>(n_mtiles * n_ntiles), static_cast<unsigned>(n_split)),
                      dim3(threads), 0, stream, t, ep);

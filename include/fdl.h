@@ -81,6 +81,8 @@ int fdl_abi_version(void);
  *            asserts that every sin/cos row repeats its first half (rope_sin[r][c + head_dim/2]
  *            == rope_sin[r][c], the same for rope_cos), as the reference's tables do
  *            (cat(freqs, freqs), generate.py:44-50); only the first half of each row is read.
+ * The sums of a row are added in an order that d_model and the column alone determine: its
+ * outputs are the same bits whatever other rows the call has.
  * Rows whose slot or rope_row is out of range are skipped by the kernel; use
  * fdl_validate_rows to reject them on the host. x, the weights, the sin/cos tables and the
  * outputs must be 16-byte aligned (d_model is a multiple of 256).
