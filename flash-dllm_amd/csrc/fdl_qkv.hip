@@ -14,23 +14,16 @@
 // computes both members of its pairs, so lane l holds (c, c + 64) of the same rows in the
 // same accumulator slot and RoPE runs in registers before the bf16 stores.
 //
-// One kernel, qkv_pc_kernel<BM, BP, NPROD, STAGES>: a workgroup computes BM rows x BP pairs
-// with wavefronts in two roles. NPROD producers move the X and W tiles of each 64-wide
-// reduction step straight from global memory into LDS (global_load_lds), STAGES steps deep;
-// four consumers (one per SIMD, a 2 x 2 grid over rows and pairs) run the 16x16x32 MFMAs
-// from LDS. A consumer never issues a global memory instruction, so its MFMA stream is
-// never held behind the texture-address queue. After the reduction the consumers stage the
-// fp32 sums in the (then free) stage memory and every wavefront rotates and writes 8-pair
-// groups with 16-byte stores. Two shapes, chosen by the number of rows (many rows run 256-row
-// tiles of another kernel, fdl_pair_gemm.h; see qkv_split):
-//  * more than 128 rows: 128 rows x 96 pairs, 4 stages of 40 KB (all of LDS). 512 rows give
-//    one tile per CU.
-//  * up to 128 rows (weight streaming, HBM-bound): 64 or 128 rows x 24 pairs (256 tiles at
-//    d_model 4096; 32 pairs beyond), 8 stages of 14 KB or 6 of 22 KB, so each workgroup keeps
-//    5-7 weight steps in flight.
+// The products run on the two kernels of the pair GEMM (fdl_pair_gemm.h), whose epilogue here
+// rotates and writes 8-pair groups with 16-byte stores. Three kinds of tiles, chosen by the
+// number of rows (qkv_split):
+//  * many rows: 256 rows x 96 pairs (pair_gemm_kernel);
+//  * more than 128 rows: 128 rows x 96 pairs, 4 stages of 40 KB, all of LDS (pair_pc_kernel).
+//    512 rows at d_model 4096 give one tile per CU;
+//  * up to 128 rows (weight streaming, HBM-bound): 64 rows x 24 or 32 pairs or 128 rows x 32
+//    pairs (pair_pc_kernel), 8 stages of 14 or 16 KB or 6 of 24 KB, so each workgroup keeps 5-7
+//    weight steps in flight.
 #include <algorithm>
-#include <atomic>
-#include <type_traits>
 
 #include "fdl_device.h"
 #include "fdl_host.h"
@@ -162,7 +155,13 @@ struct RopeEp {
   __device__ __forceinline__ const uint16_t* wrow(int p, int hi) const {
     const int pairs_per_mat = a.n_heads * kHalf;
     const int mat = p / pairs_per_mat, rem = p - mat * pairs_per_mat;
-    return a.w[mat] + int64_t((rem >> 6) * kHeadDim + (rem & 63) + kHalf * hi) * a.d_model;
+    // differences of the uniform pointers: an index that differs by lane would read the pointer
+    // from the kernel arguments in memory, and each wait for it delays the first loads
+    const uint64_t w0 = reinterpret_cast<uint64_t>(a.w[0]), w1 = reinterpret_cast<uint64_t>(a.w[1]),
+                   w2 = reinterpret_cast<uint64_t>(a.w[2]);
+    const uint64_t w = w0 + (mat >= 1 ? w1 - w0 : 0) + (mat >= 2 ? w2 - w1 : 0);
+    return reinterpret_cast<const uint16_t*>(w) +
+           int64_t((rem >> 6) * kHeadDim + (rem & 63) + kHalf * hi) * a.d_model;
   }
   __device__ __forceinline__ Row row(int64_t r) const {
     int64_t dq, dkv, rope;
@@ -196,15 +195,18 @@ struct QkvSplit {
   int64_t wide, mid;
 };
 
-// Up to 128 rows the projection streams the weights (24- or 32-pair tiles, 6-8 stages; 128 x
-// 32-pair tiles take 45 us at 192 rows against 36 us for the 128 x 96-pair ones). Beyond, two shapes feed the MFMAs: a round of 256-row tiles (80
-// us at d_model 4096, one workgroup per CU) covers as much as two rounds of 128-row tiles (47
-// us each), so whole rounds go to the 256-row tiles and a part of a round to what covers it
-// soonest: 512 rows to 128-row tiles (54 us; 256-row tiles fill half of the device and take
+// Up to 128 rows the projection streams the weights (128 x 32-pair tiles take 45 us at 192 rows
+// against 36 us for the 128 x 96-pair ones). Beyond, two shapes feed the MFMAs: a round of 256-row
+// tiles (80 us at d_model 4096, one workgroup per CU) covers as much as two rounds of 128-row
+// tiles (47 us each), so whole rounds go to the 256-row tiles and a part of a round to what covers
+// it soonest: 512 rows to 128-row tiles (54 us; 256-row tiles fill half of the device and take
 // 75), 1024 rows to 256-row tiles (100 -> 86 us), 1536 rows a round of each (140 -> 130 us), 576
 // rows a round of 128-row tiles and a 64-row stream (69 us; 256-row tiles 76), 640 rows to
 // 256-row tiles (95 -> 76 us). The split with the smallest sum is taken; a launch counts as
-// kLaunchUs.
+// kLaunchUs. At other widths the rounds' costs keep their proportions: over 147 row counts at
+// d_model 512 to 8192, timed against every other split, the choice was within 1.6% of the fastest
+// but for five (2-6%), and costs scaled with d_model beside a fixed launch choose differently at
+// four, by 2% at most.
 constexpr int kWideRoundUs = 80, kMidRoundUs = 47, kLaunchUs = 4;
 constexpr int kStreamUs[2] = {17, 21};  // up to 64 rows, up to 128
 constexpr int kStreamRows = 128;
@@ -349,15 +351,20 @@ extern "C" int fdl_qkv_rope_cache(const void* x, const void* wq, const void* wk,
     FDL_HIP_CHECK((qkv_launch_pc<kPcBM, kPcBP, 4, 4, 2>(qkv_rows(args, split.wide, split.mid), st)));
   if (rest > 0) {
     const QkvArgs tail = qkv_rows(args, split.wide + split.mid, rest);
-    // 24-pair tiles while they are one round of workgroups (d_model 4096: all 256 CUs instead of
-    // the 192 that 32-pair tiles occupy), with two producers, which load as fast as more: cold
-    // weights, 40 rows 23.0 -> 21.5 us, 64 rows 25.0 -> 23.0, 100 rows 29.2 -> 28.3; d_model 2048,
-    // 64 rows 13.5 -> 12.6
-    const bool narrow = n_heads * 3 * kHalf / 24 <= pg_device_cus();
-    FDL_HIP_CHECK((rest <= 64 ? (narrow ? qkv_launch_pc<64, 24, 2, 8, 4>(tail, st)
-                                        : qkv_launch_pc<64, 32, 4, 8, 2>(tail, st))
-                              : (narrow ? qkv_launch_pc<128, 24, 2, 6, 4>(tail, st)
-                                        : qkv_launch_pc<128, 32, 4, 6, 2>(tail, st))));
+    // Up to 64 rows 24-pair tiles, with two producers, which load as fast as more, where they are
+    // one round of workgroups on more than half of the CUs (d_model 4096: all 256, against the 192
+    // of 32-pair tiles). Before / with them, cold and warm weights (us): d_model 4096, 40 rows 22.1
+    // -> 20.9, 17.7 -> 18.3, 64 rows 24.8 -> 23.1, 18.1 -> 18.7; 2560, 64 rows 17.9 -> 17.3, 12.8 ->
+    // 12.1; but 2048, warm, 64 rows 9.7 -> 10.2 (cold 13.5 -> 12.8) and 1024 7.0 -> 7.3. Of 65
+    // to 128 rows they lose more warm than they gain cold (100 rows 19.5 -> 21.1, cold 29.2 -> 28.3;
+    // 2048: 10.7 -> 12.3, cold 16.0 -> 15.8).
+    const int64_t cus = pg_device_cus(), tiles = n_heads * 3 * kHalf / 24;
+    if (rest > 64)
+      FDL_HIP_CHECK((qkv_launch_pc<128, 32, 4, 6, 2>(tail, st)));
+    else if (2 * tiles > cus && tiles <= cus)
+      FDL_HIP_CHECK((qkv_launch_pc<64, 24, 2, 8, 4>(tail, st)));
+    else
+      FDL_HIP_CHECK((qkv_launch_pc<64, 32, 4, 8, 2>(tail, st)));
   }
   return ok();
 }
