@@ -473,21 +473,32 @@ def silu_mul(gate: torch.Tensor, up: torch.Tensor, out: torch.Tensor | None = No
     return out
 
 
-def gate_up_silu_pays(rows: int, width: int, device: torch.device) -> bool:
-    """Whether gate_up_silu is faster than one library product over both weights and silu_mul:
-    while its 128-row tiles fit one round of workgroups (width 12288: up to 256 rows; 64 rows
-    50 -> 37 us, 256 rows 67 -> 61 us), and where its 256-row tiles make one to three whole rounds
-    and are at least 25/32 full of rows (400-512 rows 98-103 -> 92-95 us, 1024 190 -> 180, 1536
-    277 -> 266; against it 384 rows 87 / 93 us, 640 rows 132 / 158, 1280 rows 220 / 246, 2048 rows
-    316 / 349)."""
-    if rows <= 0:
-        return False
+def gate_up_silu_pays(rows: int, width: int, device: torch.device, k: int = 4096) -> bool:
+    """Whether gate_up_silu over a reduction of k is faster than one library product over both
+    weights and silu_mul. Measured, library / fused (us), cold weights:
+
+    * up to 128 rows where the 48-pair tiles fit one round of workgroups or fill the last one to
+      half (k 4096, width 12288: 64 rows 49.6 / 36.9; 3072: 28.6 / 27.4; k 1024, width 3072: 14.7 /
+      8.4; k 6144, width 18432, 384 tiles on 256 CUs: 118.8 / 98.2; but k 5120, width 15360, 320
+      tiles: 62.5 / 88.4);
+    * while the 128-row tiles fit one round and occupy enough of the device, the more the longer
+      the reduction, since the library splits those: k 4096 three quarters (width 12288, 256 rows
+      69.4 / 57.1; 3072, 800 rows 50.2 / 42.4, but 640 rows 44.8 / 48.8), 2048 half (width 6144, 256
+      rows 31.7 / 30.0), 1024 any (width 3072, 160 rows 16.2 / 16.4, but 20 us less on the host);
+      and divide over the XCDs, whose L2s their row blocks share (width 8160, 384 rows 36.7 / 40.6);
+    * where the 256-row tiles make one to three whole rounds and are full enough: two of them
+      25/32 (width 12288, 400 rows 88.8 / 82.3, 512 94.8 / 88.9), more 7/8 (896 rows 181 / 172, 1024
+      185 / 176, 1400 269 / 257, but 800 rows 154 / 169; k 8192, 1400 rows 491 / 480, 896 rows 321 /
+      325), for k up to 2048 13/16 (width 6144, 832 rows 48.5 / 45.2, but 800 rows 45.6 / 45.5)."""
     cus, n_tiles = _cus(device), width // 96
-    if -(-rows // 128) * n_tiles <= cus:
-        return True
+    if rows <= 128:
+        return rows > 0 and (2 * n_tiles <= cus or (2 * n_tiles - 1) % cus + 1 >= cus // 2)
+    tiles = -(-rows // 128) * n_tiles
+    if tiles <= cus:
+        return tiles % 8 == 0 and 8 * tiles >= cus * (6 if k > 2048 else 4 if k > 1024 else 0)
     m_tiles = -(-rows // 256)
     return (m_tiles * n_tiles % cus == 0 and m_tiles * n_tiles <= 3 * cus
-            and rows >= 200 * m_tiles)
+            and rows >= m_tiles * (200 if m_tiles <= 2 else 224 if k > 2048 else 208))
 
 
 def gate_up_silu(x: torch.Tensor, w_gate: torch.Tensor, w_up: torch.Tensor,

@@ -173,10 +173,13 @@ def _plain_linear(m) -> bool:
 # compute unit. attn_out with the norm behind it, cold weights (us), library product / parts:
 # d_model 4096: 16 rows 19.5 / 14.4, 64 rows 19.8 / 15.6, 128 rows 28.7 / 18.8, 256 rows 27.0 /
 # 23.2 (512 rows: as many tiles as the library's); d_model 2048: 64 rows 12.0 / 10.0, 128 rows
-# 11.7 / 11.8, 256 rows 13.0 / 14.6. ff_out (k 12288) with the residual pass: 16 rows 26.5 / 26.2,
-# 64 rows 30.2 / 28.4, 128 rows 39.0 / 36.6, 256 rows 51 / 55; k 6144, d_model 2048: 16 rows 11.8 /
-# 14.0, 128 rows 16.3 / 21.3 (the library's four parts suffice). Each product also saves about
-# 10 us of library set-up on the host.
+# 11.7 / 11.8, 256 rows 13.0 / 14.6; 5120: 64 rows 25.9 / 22.5, 256 rows 55 / 43; 8192: 64 rows
+# 37.2 / 33.3, 256 rows 82 / 60. ff_out (k 12288) with the residual pass: 1 row 23.4 / 24.1, 16 rows
+# 26.5 / 26.2, 64 rows 30.2 / 28.4, 128 rows 39.0 / 36.6, 256 rows 51 / 55; k 6144, d_model 2048: 16
+# rows 11.8 / 14.0, 128 rows 16.3 / 21.3 (the library's four parts suffice); k 15360, d_model 5120:
+# 64 rows 62.8 / 43.6, and of more than 64 rows, where the device no longer holds eight parts, 100
+# rows 53.2 / 58.0 (8192: 82.9 / 91.4). Each product also saves about 10 us of library set-up on
+# the host.
 PARTS_MAX_ROWS = 128
 PARTS_WIDE_WEIGHT = 1 << 24          # elements from which attn_out takes twice the rows
 PARTS_FF_OUT_WEIGHT = 1 << 25        # elements from which ff_out runs in parts
@@ -197,7 +200,8 @@ def _ff_out_in_parts(w: torch.Tensor, rows: int) -> bool:
     """For an ff_out that the split-K product takes (weight stored transposed)."""
     n_out, k = w.shape
     return (rows <= PARTS_MAX_ROWS and n_out * k >= PARTS_FF_OUT_WEIGHT and k % 64 == 0
-            and n_out % 128 == 0 and w.data_ptr() % 16 == 0)
+            and n_out % 128 == 0 and w.data_ptr() % 16 == 0
+            and (rows <= 64 or n_out // 128 * 8 <= ops._cus(w.device)))
 
 
 def _fused_gate_up(x: torch.Tensor, w_gu: torch.Tensor) -> bool:
@@ -207,7 +211,7 @@ def _fused_gate_up(x: torch.Tensor, w_gu: torch.Tensor) -> bool:
     return (x.dim() == 2 and x.is_cuda and x.is_contiguous() and w_gu.dtype == torch.bfloat16
             and width % 96 == 0 and k % 128 == 0 and 256 <= k <= 65536
             and x.data_ptr() % 16 == 0 and w_gu.data_ptr() % 16 == 0
-            and ops.gate_up_silu_pays(x.shape[0], width, x.device))
+            and ops.gate_up_silu_pays(x.shape[0], width, x.device, k))
 
 
 # ff_out (K = mlp width, N = d_model) as a split-K product at up to SPLIT_K_MAX_ROWS rows:

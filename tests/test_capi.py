@@ -279,6 +279,46 @@ def test_attention_workspace_sizes():
     assert ops.attention_workspace_floats(mixed, 32) == 2 * 32 * 30 * lib.ATTN_WS_FLOATS_PER_BLOCK
 
 
+def test_gate_up_rule_follows_the_measured_sides(monkeypatch):
+    """Row counts and widths at which the fused gate and up product was measured faster (True)
+    and slower than the library's (False), on 256 compute units."""
+    from fdl import ops
+    monkeypatch.setattr(ops, "_cus", lambda dev: 256)
+    sides = {
+        (4096, 12288): {1: True, 128: True, 129: True, 256: True, 257: False, 384: False, 400: True,
+                        512: True, 640: False, 800: False, 832: False, 896: True, 1024: True,
+                        1281: False, 1400: True, 1536: True, 1900: False, 2048: False},
+        (4096, 3072): {128: True, 160: False, 512: False, 640: False, 800: True, 1024: True},
+        (4096, 10752): {256: True, 300: False, 512: False, 1024: False},
+        (2048, 6144): {256: True, 512: True, 640: False, 800: False, 832: True, 1024: True, 1300: False,
+                       1900: True, 2900: True},
+        (2048, 8160): {128: True, 256: False, 257: False, 384: False},
+        (1024, 3072): {384: True, 640: True, 1024: True, 1900: True},
+        (5120, 15360): {1: False, 64: False, 128: False},
+        (6144, 18432): {1: True, 64: True, 128: True},
+        (8192, 24576): {1: True, 128: True, 256: True, 512: True, 640: False},
+        (8192, 12288): {256: True, 512: True, 800: False, 1024: True, 1281: False, 1400: True},
+    }
+    for (k, width), rows in sides.items():
+        for r, pays in rows.items():
+            assert ops.gate_up_silu_pays(r, width, None, k) is pays, (k, width, r)
+
+
+def test_ff_out_parts_rule_follows_the_measured_sides(monkeypatch):
+    """Where ff_out runs in parts on 256 compute units: large weights, up to 128 rows, beyond 64
+    only while the device holds eight parts at once."""
+    import torch
+    import flash_cache_hip as fch
+    from fdl import ops
+    monkeypatch.setattr(ops, "_cus", lambda dev: 256)
+    for n_out, k, rows in ((4096, 12288, {64: True, 100: True, 128: True, 129: False}),
+                           (5120, 15360, {64: True, 65: False, 100: False}),
+                           (8192, 24576, {64: True, 100: False}), (2048, 6144, {16: False, 128: False})):
+        w = torch.empty((n_out, k), dtype=torch.bfloat16, device="meta")
+        for r, parts in rows.items():
+            assert fch._ff_out_in_parts(w, r) is parts, (n_out, k, r)
+
+
 def test_validate_work():
     pt = contiguous_page_table(2, 128)
     work, rows, n_long, n_mid = build_work([SeqRows(0, 100, np.arange(0, 40), 8),
