@@ -29,7 +29,7 @@ __device__ __forceinline__ float round_bf(float f) { return bf2f(f2bf(f)); }
 // order and rounded to bf16 first.
 enum class Residual { kNone, kRows, kPartials };
 template <Residual kRes>
-__global__ __launch_bounds__(kNormThreads) void rms_norm_kernel(
+__device__ __forceinline__ void rms_norm_row(
     const uint16_t* __restrict__ x, const uint16_t* __restrict__ res,
     const float* __restrict__ part, int n_split, int64_t stride,
     const uint16_t* __restrict__ w, int d, float eps, uint16_t* __restrict__ sum_out,
@@ -99,6 +99,24 @@ __global__ __launch_bounds__(kNormThreads) void rms_norm_kernel(
       st16(out + row * d + 8 * c, o);
     }
   }
+}
+
+// A kernel for each kind of residual, so that none is launched with arguments it has no use for
+// (8 rows of 4096: 2.95 us with the partial sums' three, 2.80 without).
+template <bool kResidual>
+__global__ __launch_bounds__(kNormThreads) void rms_norm_kernel(
+    const uint16_t* __restrict__ x, const uint16_t* __restrict__ res,
+    const uint16_t* __restrict__ w, int d, float eps, uint16_t* __restrict__ sum_out,
+    uint16_t* __restrict__ out) {
+  rms_norm_row<kResidual ? Residual::kRows : Residual::kNone>(x, res, nullptr, 0, 0, w, d, eps,
+                                                              sum_out, out);
+}
+
+__global__ __launch_bounds__(kNormThreads) void rms_norm_partials_kernel(
+    const uint16_t* __restrict__ x, const float* __restrict__ part, int n_split, int64_t stride,
+    const uint16_t* __restrict__ w, int d, float eps, uint16_t* __restrict__ sum_out,
+    uint16_t* __restrict__ out) {
+  rms_norm_row<Residual::kPartials>(x, nullptr, part, n_split, stride, w, d, eps, sum_out, out);
 }
 
 constexpr int kEwThreads = 256;
@@ -214,10 +232,9 @@ extern "C" int fdl_rms_norm(const void* x, const void* residual, const void* wei
   const auto* wp = static_cast<const uint16_t*>(weight);
   auto* sp = static_cast<uint16_t*>(sum_out);
   auto* op = static_cast<uint16_t*>(out);
-  hipLaunchKernelGGL((residual ? rms_norm_kernel<Residual::kRows> : rms_norm_kernel<Residual::kNone>),
-                     dim3(static_cast<unsigned>(n_rows)), dim3(kNormThreads), 0, st, xp, rp,
-                     static_cast<const float*>(nullptr), 0, int64_t(0), wp, static_cast<int>(d),
-                     eps, sp, op);
+  hipLaunchKernelGGL((residual ? rms_norm_kernel<true> : rms_norm_kernel<false>),
+                     dim3(static_cast<unsigned>(n_rows)), dim3(kNormThreads), 0, st, xp, rp, wp,
+                     static_cast<int>(d), eps, sp, op);
   FDL_HIP_CHECK(hipGetLastError());
   return ok();
 }
@@ -245,9 +262,9 @@ extern "C" int fdl_rms_norm_partials(const void* x, const float* part, int64_t n
   FDL_REQUIRE_ALIGNED(weight, 16);
   FDL_REQUIRE_ALIGNED(sum_out, 16);
   FDL_REQUIRE_ALIGNED(out, 16);
-  hipLaunchKernelGGL(rms_norm_kernel<Residual::kPartials>, dim3(static_cast<unsigned>(n_rows)),
+  hipLaunchKernelGGL(rms_norm_partials_kernel, dim3(static_cast<unsigned>(n_rows)),
                      dim3(kNormThreads), 0, static_cast<hipStream_t>(stream),
-                     static_cast<const uint16_t*>(x), static_cast<const uint16_t*>(nullptr), part,
+                     static_cast<const uint16_t*>(x), part,
                      static_cast<int>(n_split), n_rows * d, static_cast<const uint16_t*>(weight),
                      static_cast<int>(d), eps, static_cast<uint16_t*>(sum_out),
                      static_cast<uint16_t*>(out));
