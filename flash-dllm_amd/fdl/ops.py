@@ -52,6 +52,19 @@ def _need(t: torch.Tensor, name: str, dtype: torch.dtype, ndim: int | None = Non
         raise _lib.FdlError(_lib.FDL_ERR_SHAPE, f"{name} must be contiguous")
 
 
+def plain_module(m, cls) -> bool:
+    """Whether calling module `m` now runs cls.forward and nothing else, so that a kernel may take
+    its place: exactly of class cls, without a forward of its own (offload and adapter wrappers
+    set one), without hooks of its own or of all modules, and not being traced or compiled or
+    under a function transform (vmap, forward-mode derivatives), which see no kernel launch."""
+    return (type(m) is cls and "forward" not in m.__dict__
+            and not (m._forward_hooks or m._forward_pre_hooks or m._backward_hooks
+                     or m._backward_pre_hooks or torch.nn.modules.module._has_any_global_hook())
+            and torch.autograd.forward_ad._current_level < 0
+            and torch._C._functorch.peek_interpreter_stack() is None
+            and not torch.jit.is_tracing() and not torch.compiler.is_compiling())
+
+
 _halves_seen: dict = {}
 
 

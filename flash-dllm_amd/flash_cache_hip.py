@@ -159,11 +159,12 @@ def _adjacent_gate_up(block) -> torch.Tensor | None:
 
 
 def _plain_linear(m) -> bool:
-    """A torch.nn.Linear with a plain contiguous bf16 GPU weight, without bias or hooks: its
-    product may run without calling the module."""
-    w = getattr(m, "weight", None)
-    return (type(m) is torch.nn.Linear and m.bias is None and not m._forward_hooks
-            and not m._forward_pre_hooks and type(w) in (torch.nn.Parameter, torch.Tensor)
+    """A torch.nn.Linear that only forms its product (ops.plain_module), with a plain contiguous
+    bf16 GPU weight, without bias and outside autocast: the product may run without a call."""
+    if not ops.plain_module(m, torch.nn.Linear) or torch.is_autocast_enabled("cuda"):
+        return False
+    w = m.weight
+    return (m.bias is None and type(w) in (torch.nn.Parameter, torch.Tensor)
             and w.dtype == torch.bfloat16 and w.is_cuda and w.is_contiguous()
             and w.data_ptr() % 16 == 0)
 

@@ -243,3 +243,64 @@ def test_final_norm_matches_module(rows):
         assert got.shape == x.shape
         _check(got, norm(x), f"final norm {rows}")
     assert _final_norm(norm, x).requires_grad
+
+
+def _elsewhere(case, m, x):
+    """A forward of `m` that must not be bypassed: sets it up, returns (calls so far, undo)."""
+    calls = []
+    if case == "forward":  # as an offload or adapter wrapper replaces it
+        own = m.forward
+        m.forward = lambda *a: (calls.append(1), own(*a))[1]
+        return calls, lambda: m.__dict__.pop("forward")
+    if case == "global hook":
+        h = torch.nn.modules.module.register_module_forward_hook(
+            lambda mod, a, out: calls.append(1) if mod is m else None)
+        return calls, h.remove
+    h = m.register_forward_pre_hook(lambda mod, a: calls.append(1))
+    return calls, h.remove
+
+
+@pytest.mark.parametrize("case", ["forward", "global hook", "hook"])
+@torch.no_grad()
+def test_modules_that_do_more_than_their_forward_are_called(case):
+    """attn_out in a block's tail and the final norm run their modules where a call does more
+    than the class's forward, and in kernels of their own again afterwards, with like results."""
+    import flash_cache_hip as fch
+    from fdl.model import LLaDAConfig, LLaDALlamaBlock, _final_norm
+    cfg = LLaDAConfig(d_model=512, n_heads=4, mlp_hidden_size=1536)
+    blk = LLaDALlamaBlock(cfg, 0, fch.flash_fused_elastic_cache, device=DEV, dtype=torch.bfloat16)
+    for p in blk.parameters():
+        p.normal_(0.0, 0.05)
+    norm = RMSLayerNorm(512, 1e-5, DEV, torch.bfloat16)
+    x, att = (torch.randn(8, 512, device=DEV).to(torch.bfloat16) for _ in range(2))
+    want = fch.block_mlp_tail(blk, x, att), _final_norm(norm, x)
+    for m, run, ref in ((blk.attn_out, lambda: fch.block_mlp_tail(blk, x, att), want[0]),
+                        (norm, lambda: _final_norm(norm, x), want[1])):
+        calls, undo = _elsewhere(case, m, x)
+        got = run()
+        undo()
+        assert len(calls) == 1
+        torch.testing.assert_close(got.float(), ref.float(), atol=2e-2, rtol=1e-2)
+        run()
+        assert len(calls) == 1
+
+
+def test_final_norm_keeps_forward_mode_derivatives_and_autocast_products():
+    """A tangent passes through the final norm as through its module; attn_out under autocast is
+    the module's product in autocast's type."""
+    import torch.autograd.forward_ad as fwd
+    import flash_cache_hip as fch
+    from fdl.model import _final_norm
+    norm = RMSLayerNorm(64, 1e-5, DEV, torch.bfloat16).requires_grad_(False)
+    x, t = (torch.randn(5, 64, device=DEV).to(torch.bfloat16) for _ in range(2))
+    with fwd.dual_level():
+        got = fwd.unpack_dual(_final_norm(norm, fwd.make_dual(x, t))).tangent
+        ref = fwd.unpack_dual(norm(fwd.make_dual(x, t))).tangent
+        assert got is not None and torch.equal(got, ref)
+    got = torch.func.vmap(lambda r: _final_norm(norm, r))(x)
+    torch.testing.assert_close(got.float(), norm(x).float(), atol=2e-2, rtol=1e-2)
+    m = torch.nn.Linear(256, 256, bias=False, device=DEV, dtype=torch.bfloat16)
+    a = torch.randn(8, 256, device=DEV).to(torch.bfloat16)
+    assert fch._attn_out_in_parts(m, a, a)
+    with torch.autocast("cuda", torch.float16):
+        assert not fch._attn_out_in_parts(m, a, a)
