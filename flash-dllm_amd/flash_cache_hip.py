@@ -187,13 +187,19 @@ PARTS_FF_OUT_WEIGHT = 1 << 25        # elements from which ff_out runs in parts
 
 
 def _attn_out_in_parts(m, x: torch.Tensor, att: torch.Tensor) -> bool:
-    if not (_plain_linear(m) and att.dim() == 2 and att.dtype == torch.bfloat16 and att.is_cuda
+    # the cheapest first: a larger call should not pay for all of them (640 rows of d_model 2048,
+    # host time of the block's tail: 102 us before there were any, 107 with these last, 103)
+    if type(m) is not torch.nn.Linear or att.dim() != 2:
+        return False
+    rows = att.shape[0]
+    if not 0 < rows <= 2 * PARTS_MAX_ROWS or (
+            rows > PARTS_MAX_ROWS and m.weight.numel() < PARTS_WIDE_WEIGHT):
+        return False
+    if not (_plain_linear(m) and att.dtype == torch.bfloat16 and att.is_cuda
             and att.is_contiguous() and att.data_ptr() % 16 == 0):
         return False
     n_out, k = m.weight.shape
-    rows = att.shape[0]
-    return (0 < rows <= PARTS_MAX_ROWS * (2 if n_out * k >= PARTS_WIDE_WEIGHT else 1)
-            and k % 64 == 0 and n_out % 128 == 0 and tuple(x.shape) == (rows, n_out)
+    return (k % 64 == 0 and n_out % 128 == 0 and tuple(x.shape) == (rows, n_out)
             and att.shape[1] == k)
 
 
@@ -209,10 +215,10 @@ def _fused_gate_up(x: torch.Tensor, w_gu: torch.Tensor) -> bool:
     """Whether the gate and up products and the SiLU gate run as one kernel
     (ops.gate_up_silu): the shapes it takes, at row counts where it is the faster way."""
     width, k = w_gu.shape[0] // 2, w_gu.shape[1]
-    return (x.dim() == 2 and x.is_cuda and x.is_contiguous() and w_gu.dtype == torch.bfloat16
-            and width % 96 == 0 and k % 128 == 0 and 256 <= k <= 65536
-            and x.data_ptr() % 16 == 0 and w_gu.data_ptr() % 16 == 0
-            and ops.gate_up_silu_pays(x.shape[0], width, x.device, k))
+    return (width % 96 == 0 and k % 128 == 0 and 256 <= k <= 65536 and x.is_cuda
+            and ops.gate_up_silu_pays(x.shape[0], width, x.device, k)
+            and x.dim() == 2 and x.is_contiguous() and w_gu.dtype == torch.bfloat16
+            and x.data_ptr() % 16 == 0 and w_gu.data_ptr() % 16 == 0)
 
 
 # ff_out (K = mlp width, N = d_model) as a split-K product at up to SPLIT_K_MAX_ROWS rows:

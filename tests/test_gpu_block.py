@@ -228,6 +228,9 @@ def test_attn_out_with_hooks_is_called_as_a_module():
     assert not fch._attn_out_in_parts(torch.nn.Linear(256, 256, device=DEV, dtype=torch.bfloat16), x, x)
     assert not fch._attn_out_in_parts(m, x, x.t().contiguous().t())
     assert not fch._attn_out_in_parts(m, x[:, :128], x)
+    many = torch.randn(200, 256, device=DEV).to(torch.bfloat16)
+    assert not fch._attn_out_in_parts(m, many, many)  # a small weight's rows
+    assert not fch._attn_out_in_parts(torch.nn.Identity(), many, many)
 
 
 @pytest.mark.parametrize("rows", [1, 37])
