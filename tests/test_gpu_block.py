@@ -233,6 +233,37 @@ def test_attn_out_with_hooks_is_called_as_a_module():
     assert not fch._attn_out_in_parts(torch.nn.Identity(), many, many)
 
 
+@pytest.mark.parametrize("rows", [1, 64, 65, 128])
+@torch.no_grad()
+def test_block_mlp_tail_with_every_product_of_few_rows(rows):
+    """The epilogue of few rows at a width whose ff_out (2^25 elements) runs in parts, beside
+    attn_out in parts and the fused gate and up product, against float32 products of the same
+    bf16 intermediates. The output is a bf16 residual stream of size ~1 plus an MLP term of about
+    that size: the roundings of g, u and their product (2^-9 of each of 18432 terms, in random
+    directions) stay far below the result's own, 2^-9 of values up to 8, and a changed rounding of
+    the residual, 2^-8 of it: 2^-7 of the value, bounded here by 2e-2."""
+    import flash_cache_hip as fch
+    from fdl.model import LLaDAConfig, LLaDALlamaBlock
+    cfg = LLaDAConfig(d_model=2048, n_heads=16, mlp_hidden_size=18432)
+    blk = LLaDALlamaBlock(cfg, 0, fch.flash_fused_elastic_cache, device=DEV, dtype=torch.bfloat16)
+    gen = torch.Generator(device=DEV).manual_seed(rows)
+    for p in blk.parameters():
+        p.normal_(0.0, 0.02, generator=gen) if p.dim() == 2 else p.normal_(1.0, 0.1, generator=gen)
+    x, att = (torch.randn(rows, 2048, generator=gen, device=DEV).to(torch.bfloat16) for _ in range(2))
+    assert fch._attn_out_in_parts(blk.attn_out, x, att)
+    assert fch._ff_out_in_parts(blk.ff_out.weight, rows) and fch._split_k_ff_out(blk, rows) is not None
+    assert fch._fused_gate_up(x, fch._adjacent_gate_up(blk))
+    x0 = x.clone()
+    got = fch.block_mlp_tail(blk, x, att)
+    assert torch.equal(x, x0) and got.shape == (1, rows, 2048)
+    og = x + (att.float() @ blk.attn_out.weight.float().t()).to(torch.bfloat16)
+    xn = blk.ff_norm(og)
+    g = torch.nn.functional.silu((xn.float() @ blk.ff_proj.weight.float().t()).to(torch.bfloat16))
+    u = (xn.float() @ blk.up_proj.weight.float().t()).to(torch.bfloat16)
+    ref = og.float() + (g * u).float() @ blk.ff_out.weight.float().t()
+    torch.testing.assert_close(got[0].float(), ref, atol=5e-2, rtol=2e-2)
+
+
 @pytest.mark.parametrize("rows", [1, 37])
 def test_final_norm_matches_module(rows):
     """The model's final norm in one kernel against the module (the bounds of the norm kernel's
