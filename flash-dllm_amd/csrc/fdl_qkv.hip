@@ -20,8 +20,8 @@
 //  * many rows: 256 rows x 96 pairs (pair_gemm_kernel);
 //  * more than 128 rows: 128 rows x 96 pairs, 4 stages of 40 KB, all of LDS (pair_pc_kernel).
 //    512 rows at d_model 4096 give one tile per CU;
-//  * up to 128 rows (weight streaming, HBM-bound): 64 rows x 24 or 32 pairs or 128 rows x 32
-//    pairs (pair_pc_kernel), 8 stages of 14 or 16 KB or 6 of 24 KB, so each workgroup keeps 5-7
+//  * up to 128 rows (weight streaming, HBM-bound): 64 or 128 rows x 24 or 32 pairs
+//    (pair_pc_kernel), 8 stages of 14 or 16 KB or 6 of 22 or 24 KB, so each workgroup keeps 5-7
 //    weight steps in flight.
 #include <algorithm>
 
@@ -351,20 +351,20 @@ extern "C" int fdl_qkv_rope_cache(const void* x, const void* wq, const void* wk,
     FDL_HIP_CHECK((qkv_launch_pc<kPcBM, kPcBP, 4, 4, 2>(qkv_rows(args, split.wide, split.mid), st)));
   if (rest > 0) {
     const QkvArgs tail = qkv_rows(args, split.wide + split.mid, rest);
-    // Up to 64 rows 24-pair tiles, with two producers, which load as fast as more, where they are
-    // one round of workgroups on more than half of the CUs (d_model 4096: all 256, against the 192
-    // of 32-pair tiles). Before / with them, cold and warm weights (us): d_model 4096, 40 rows 22.1
-    // -> 20.9, 17.7 -> 18.3, 64 rows 24.8 -> 23.1, 18.1 -> 18.7; 2560, 64 rows 17.9 -> 17.3, 12.8 ->
-    // 12.1; but 2048, warm, 64 rows 9.7 -> 10.2 (cold 13.5 -> 12.8) and 1024 7.0 -> 7.3. Of 65
-    // to 128 rows they lose more warm than they gain cold (100 rows 19.5 -> 21.1, cold 29.2 -> 28.3;
-    // 2048: 10.7 -> 12.3, cold 16.0 -> 15.8).
+    // 24-pair tiles, with two producers, which load as fast as more, where they are one round of
+    // workgroups on more than half of the CUs (d_model 4096: all 256, against the 192 of 32-pair
+    // tiles), and of 65 to 128 rows on more than 7/8. Without / with them, cold and warm weights
+    // (us): d_model 4096, 40 rows 22.1 -> 20.9, 17.7 -> 18.3, 64 rows 24.8 -> 23.1, 18.1 -> 18.7, 100
+    // rows 29.5 -> 28.3, 19.5 -> 21.1; 2560, 64 rows 17.9 -> 17.3, 12.8 -> 12.1. A model's weights are
+    // cold: its other layers come between. Elsewhere they lose more than that warm: 2048, 64 rows
+    // 13.5 -> 12.8, 9.7 -> 10.2, 100 rows 16.0 -> 15.8, 10.7 -> 12.3; 3072, 65 rows 21.1 -> 19.9, 14.6
+    // -> 15.8; 1024, 64 rows 8.7 -> 8.4, 7.0 -> 7.3.
     const int64_t cus = pg_device_cus(), tiles = n_heads * 3 * kHalf / 24;
-    if (rest > 64)
-      FDL_HIP_CHECK((qkv_launch_pc<128, 32, 4, 6, 2>(tail, st)));
-    else if (2 * tiles > cus && tiles <= cus)
-      FDL_HIP_CHECK((qkv_launch_pc<64, 24, 2, 8, 4>(tail, st)));
-    else
-      FDL_HIP_CHECK((qkv_launch_pc<64, 32, 4, 8, 2>(tail, st)));
+    const bool narrow = tiles <= cus && (rest <= 64 ? 2 * tiles > cus : 8 * tiles > 7 * cus);
+    FDL_HIP_CHECK((rest <= 64 ? (narrow ? qkv_launch_pc<64, 24, 2, 8, 4>(tail, st)
+                                        : qkv_launch_pc<64, 32, 4, 8, 2>(tail, st))
+                              : (narrow ? qkv_launch_pc<128, 24, 2, 6, 4>(tail, st)
+                                        : qkv_launch_pc<128, 32, 4, 6, 2>(tail, st))));
   }
   return ok();
 }
