@@ -59,17 +59,19 @@ struct PairGemmTiles {
   int start_mul;  // see pg_start
 };
 
-// The reduction step that the tile of pairs p0 .. starts its walk with (it wraps around). When all
-// workgroups read the same 128 bytes of their weight rows (a power of two apart) at a time, the
-// reads crowd on few HBM channels; cold weights, all in step / started apart: gate and up at 64
-// rows (201 MB) 46.8 / 36.9 us, at 128 rows 50.9 / 43.4, the 40-row projection (101 MB) 24.1 /
-// 22.1. The pairs are cut into groups of kPgStartPairs, a multiple of every tile's width, and the
-// groups spread over kPgStarts even places (8 places: 128 rows of gate and up 45.4 us; 32 or 64
-// no better than 16). The place depends on the pair and the number of pairs alone, so a row's
+// The reduction step that the tile of pairs p0 .. starts its walk with (it wraps around). Where the
+// weight rows are a multiple of 4 KB apart and all workgroups read the same 128 bytes of them at a
+// time, the reads crowd on few HBM channels; cold weights, all in step / started apart (us): rows
+// of 8 KB, gate and up of 64 rows (201 MB) 44.6 / 36.8, of 128 rows 47.9 / 42.1, the 40-row
+// projection (101 MB) 23.5 / 20.8; rows of 4 KB, gate and up of one row 13.4 / 11.7, of 128 rows
+// 18.0 / 17.3; other distances (2, 5, 6, 7 KB) the same within 1%, so those start in step. The pairs
+// are cut into groups of kPgStartPairs, a multiple of every tile's width, and the groups spread
+// over kPgStarts even places (8 places: 128 rows of gate and up 45.4 us; 32 or 64 no better than
+// 16). The place depends on the pair, the number of pairs and the rows' length alone, so a row's
 // sums are added in the same order, and are the same bits, whatever the number of rows and the
 // tile. Launches of many row blocks gain nothing from it and lose nothing (6842 rows of the
 // projection 544 / 547 us).
-constexpr int kPgStartPairs = 96, kPgStarts = 16;
+constexpr int kPgStartPairs = 96, kPgStarts = 16, kPgStartStride = 2048;  // (elements)
 __device__ __forceinline__ int pg_start(const PairGemmTiles& t, int p0, int nk) {
   return ((p0 / kPgStartPairs * t.start_mul) >> 16) * nk / kPgStarts;
 }
@@ -594,7 +596,7 @@ hipError_t pair_launch(void (*kernel)(PairGemmTiles, Ep), int bm, int bp, int th
   const int64_t groups = (n_pairs + kPgStartPairs - 1) / kPgStartPairs;
   const PairGemmTiles t = {x, n_rows, static_cast<int>(k / n_split), static_cast<int>(n_mtiles),
                            static_cast<int>(n_ntiles), static_cast<int>(k),
-                           static_cast<int>((kPgStarts << 16) / groups)};
+                           k % kPgStartStride ? 0 : static_cast<int>((kPgStarts << 16) / groups)};
   hipLaunchKernelGGL(kernel,
                      dim3(static_cast<unsigned>(n_mtiles * n_ntiles), static_cast<unsigned>(n_split)),
                      dim3(threads), 0, stream, t, ep);
