@@ -133,10 +133,11 @@ __global__ __launch_bounds__(kDirectThreads) void softmax_conf_direct_kernel(
 // against 43.0 at 256 x 126464 N(0, 200^2) values, 12.2 against 9.7 at 32 x 16384 N(0, 40^2)).
 // Measured (us), each exponential computed / tabulated: 256 rows of 126464 69.9 / 19.6, 32 rows
 // 57.7 / 19.3, 512 rows of 32000 30.9 / 20.1; of a second pass: 256 rows of 126464 70.0 / 43.0,
-// of 32000 16.5 / 15.3, of 16384 10.0 / 10.4, the one place that loses. What is left are the look-ups (random 8-byte LDS reads) and
-// their addresses: one row alone takes 18 us. Below 16384 values the table costs more than it
-// saves (512 rows of 8192: 10.0 computed, 14 tabulated; of 16384: 16.9 and 16.4), so shorter rows
-// keep the direct kernel.
+// of 32000 16.5 / 15.3, of 16384 10.0 / 10.4, the one place that loses. What is left are the
+// look-ups (random 8-byte LDS reads: the LDS is active a quarter of the cycles, 59% of that in
+// bank conflicts, and wavefronts wait half of theirs) and their addresses: one row alone takes 17
+// us. Below 16384 values the table costs more than it saves (512 rows of 8192: 10.0 computed, 14
+// tabulated; of 16384: 16.9 and 16.4), so shorter rows keep the direct kernel.
 constexpr int64_t kTableVocab = 16384;
 
 // exp of the bf16 values with |x| in [2^-10, 2^6) (16 exponents, both signs) from a table of

@@ -259,14 +259,14 @@ hipError_t gu_pc(const GuCall& c, int64_t n) {
                      c.stream);
 }
 
-// Up to 128 rows the weights stream: 24 pairs a workgroup while that is one round of
-// workgroups (width 6144 at 64 rows: 13.4 us, 32 pairs 14.5), else 48 (width 12288: 256
-// workgroups; 32 pairs make one and a half rounds, 51.6 us at 64 rows against 46.4). Then 128-row tiles while they fit one round (256 rows of width
-// 12288: 61 us, 256-row tiles 85), then 256-row tiles. Against a library product over both
-// weights and a separate SiLU pass, k 4096, width 12288, cold weights (us): 64 rows 50.3 -> 37.1,
-// 128 rows 53.5 -> 45.3, 256 rows 67 -> 61, 512 rows 98 -> 95, 1024 rows 190 -> 180; 384 rows 87
-// against 93, 640 rows 132 against 158, 1900 rows 308 against 330: a caller gains while the
-// 128-row tiles fit one round and where the 256-row tiles fill whole ones.
+// Up to 128 rows the weights stream: 24 pairs a workgroup while that is one round of workgroups
+// (width 6144 at 64 rows: 13.4 us, 32 pairs 14.5), else 48 (width 12288: 256 workgroups; 32 pairs
+// make one and a half rounds, 51.6 us at 64 rows against 46.4, before the starts were spread).
+// Then 128-row tiles while they fit one round (256 rows of width 12288: 57 us, 256-row tiles 85),
+// then 256-row tiles. Against a library product over both weights and a separate SiLU pass, k
+// 4096, width 12288, cold weights (us): 64 rows 49.6 -> 36.9, 128 rows 52.9 -> 42.5, 256 rows 69 ->
+// 57, 512 rows 95 -> 89, 1024 rows 185 -> 176; 384 rows 84 against 86, 640 rows 130 against 157,
+// 1900 rows 316 against 340: a caller gains while the tiles fill their rounds.
 hipError_t gu_launch(const GuCall& c, int64_t n) {
   const int64_t cus = pg_device_cus();
   if (n <= 128) {

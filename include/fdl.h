@@ -339,7 +339,9 @@ int fdl_split_reduce_residual(const float* part, int64_t n_split, int64_t n_rows
  *                  arg[r] (if arg != NULL) = the first index of the row's maximum logit;
  *   token != NULL: prob[r] = softmax(logits[r].to(float64))[token[r]] (generate.py:337),
  *                  0 for a token outside [0, vocab); arg[r] as above if arg != NULL.
- * The float64 terms are the same as torch's; the order of the float64 sum differs.
+ * The float64 terms are torch's, exp(x - max), or with many logits exp(x), their sum divided by
+ * exp(max); the order of the float64 sum differs. No probability exceeds 1, and a row whose
+ * maximum holds everything has exactly 1.
  */
 int fdl_softmax_confidence(const void* logits, int64_t n_rows, int64_t vocab,
                            const int64_t* token, double* prob, int64_t* arg, void* stream);
